@@ -28,6 +28,7 @@ UNITS = {
     "k_fine.hip": [],
     "k_fine_modal.hip": [],
     "k_coarse.hip": [],
+    "k_dense.hip": [],
     "k_galerkin.hip": [],
     "k_simp.hip": [],
     "k_worst.hip": [],
@@ -64,7 +65,7 @@ def build_library(jobs=None):
                 print(f"[build] {futs[f]}: {err}", file=sys.stderr)
             objs.append(obj)
     tmp = LIB + ".tmp"
-    cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp] + sorted(objs) + ["-lrocsolver", "-lrocblas"]
+    cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp] + sorted(objs) + ["-lrocblas"]
     p = subprocess.run(cmd, capture_output=True, text=True)
     if p.returncode != 0:
         raise RuntimeError("link failed:\n" + p.stderr)

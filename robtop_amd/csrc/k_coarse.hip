@@ -802,11 +802,12 @@ __global__ void k_gather_rows(const int* __restrict__ rowslot, int nrows, Vec3<c
 }
 
 template <typename T>
-__global__ void __launch_bounds__(64) k_dense_gemv(const double* __restrict__ A, int n, const double* __restrict__ f,
-                                                   const int* __restrict__ rowslot, Vec3<T> U) {
+__global__ void __launch_bounds__(64) k_dense_gemv(const double* __restrict__ A, int n, int ld,
+                                                   const double* __restrict__ f, const int* __restrict__ rowslot,
+                                                   Vec3<T> U) {
     const int row = blockIdx.x;
     double s = 0;
-    const double* a = A + (size_t)row * n;
+    const double* a = A + (size_t)row * ld;
     for (int j = threadIdx.x; j < n; j += 64) s += a[j] * f[j];
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
@@ -814,12 +815,13 @@ __global__ void __launch_bounds__(64) k_dense_gemv(const double* __restrict__ A,
 }
 
 template <typename T>
-void launch_coarsest(const double* Ainv, int n3, const int* rowslot, int, Vec3<const T> F, Vec3<T> U, double* fbuf,
+void launch_coarsest(const double* Ainv, int n3, const int* rowslot, Vec3<const T> F, Vec3<T> U, double* fbuf,
                      hipStream_t s) {
     const int nrows = n3 / 3;
     if (nrows <= 0) return;
     hipLaunchKernelGGL((k_gather_rows<T>), dim3((nrows + 255) / 256), dim3(256), 0, s, rowslot, nrows, F, fbuf);
-    hipLaunchKernelGGL((k_dense_gemv<T>), dim3(n3), dim3(64), 0, s, Ainv, n3, (const double*)fbuf, rowslot, U);
+    hipLaunchKernelGGL((k_dense_gemv<T>), dim3(n3), dim3(64), 0, s, Ainv, n3, dense_ld(n3), (const double*)fbuf,
+                       rowslot, U);
     RT_HIP(hipGetLastError());
 }
 
@@ -836,40 +838,32 @@ void launch_to_bf16(const double* a, bf16* b, size_t n, hipStream_t s) {
     RT_HIP(hipGetLastError());
 }
 
-// A[r][c] = A[c][r] for c < r (row-major n x n): completes a symmetric matrix
-// whose upper triangle holds the values
-__global__ void k_mirror_upper(double* __restrict__ A, int n) {
-    const int r = blockIdx.y;
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < r; c += gridDim.x * blockDim.x)
-        A[(size_t)r * n + c] = A[(size_t)c * n + r];
-}
-void launch_mirror_upper(double* A, int n, hipStream_t s) {
-    hipLaunchKernelGGL(k_mirror_upper, dim3((n + 255) / 256, n), dim3(256), 0, s, A, n);
-    RT_HIP(hipGetLastError());
-}
-
-// dense n x n (n = 3 nr) matrix of a level from its FP64 stencils: row block r
-// (slot slots[r]) takes neighbour nb's 3 x 3 block at column block
-// nbcol[27 r + nb] (-1: outside the box or inactive). A must be zero on entry.
+// dense matrix of a level from its FP64 stencils, n = 3 nr, row stride ld =
+// dense_ld(n): row block r (slot slots[r]) takes neighbour nb's 3 x 3 block at
+// column block nbcol[27 r + nb] (-1: outside the box or inactive); the ld - n
+// padding unknowns get a unit diagonal. A must be zero on entry.
 __global__ void k_dense_from_stencil(const double* __restrict__ st, size_t N, const int* __restrict__ slots,
-                                     const int* __restrict__ nbcol, int nr, double* __restrict__ A) {
-    const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-    if (i >= (size_t)nr * 243) return;
+                                     const int* __restrict__ nbcol, int nr, int ld, double* __restrict__ A) {
+    const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x, ne = (size_t)nr * 243;
+    if (i >= ne) {
+        const size_t d = 3 * (size_t)nr + (i - ne);
+        if (d < (size_t)ld) A[d * ld + d] = 1.0;
+        return;
+    }
     const int r = (int)(i / 243), k = (int)(i % 243);
     const int nb = k / 9, a = k % 9 / 3, b = k % 3;
     const int c = nbcol[27 * r + nb];
     if (c < 0) return;
-    const size_t n = 3 * (size_t)nr;
-    A[(3 * (size_t)r + a) * n + 3 * (size_t)c + b] = st[(size_t)k * N + slots[r]];
+    A[(3 * (size_t)r + a) * ld + 3 * (size_t)c + b] = st[(size_t)k * N + slots[r]];
 }
 void launch_dense_from_stencil(const double* st, size_t N, const int* slots, const int* nbcol, int nr, double* A,
                                hipStream_t s) {
-    const size_t n = 3 * (size_t)nr;
-    RT_HIP(hipMemsetAsync(A, 0, sizeof(double) * n * n, s));
-    const size_t work = (size_t)nr * 243;
-    if (work == 0) return;
+    const int ld = dense_ld(3 * nr);
+    RT_HIP(hipMemsetAsync(A, 0, sizeof(double) * ld * (size_t)ld, s));
+    if (nr <= 0) return;
+    const size_t work = (size_t)nr * 243 + (size_t)(ld - 3 * nr);
     hipLaunchKernelGGL(k_dense_from_stencil, dim3((unsigned)((work + 255) / 256)), dim3(256), 0, s, st, N, slots,
-                       nbcol, nr, A);
+                       nbcol, nr, ld, A);
     RT_HIP(hipGetLastError());
 }
 
@@ -1276,8 +1270,7 @@ RT_INST_CS(float, bf16)
                                      const uint8_t*, int, T*, hipStream_t);                                           \
     template void launch_prolong<T>(const Geom&, const int*, Vec3<T>, const uint8_t*, const Geom&, const int*,        \
                                     Vec3<const T>, int, bool, hipStream_t);                                           \
-    template void launch_coarsest<T>(const double*, int, const int*, int, Vec3<const T>, Vec3<T>, double*,            \
-                                     hipStream_t);                                                                    \
+    template void launch_coarsest<T>(const double*, int, const int*, Vec3<const T>, Vec3<T>, double*, hipStream_t);   \
     template void launch_fill<T>(T*, T, size_t, hipStream_t);                                                         \
     template void launch_box_to_oct<T>(const Geom&, const T*, T*, int, hipStream_t);                                  \
     template void launch_oct_to_box<T>(const Geom&, const T*, T*, int, hipStream_t);
@@ -1534,14 +1527,14 @@ __global__ void k_gather_rows_b(const int* __restrict__ rowslot, int nrows, cons
 }
 
 template <typename T>
-__global__ void __launch_bounds__(64) k_dense_gemv_b(const double* __restrict__ A, int n, const double* __restrict__ f,
-                                                     const int* __restrict__ rowslot, T* __restrict__ U, int N, int bs,
-                                                     int nb) {
+__global__ void __launch_bounds__(64) k_dense_gemv_b(const double* __restrict__ A, int n, int ld,
+                                                     const double* __restrict__ f, const int* __restrict__ rowslot,
+                                                     T* __restrict__ U, int N, int bs, int nb) {
     const int row = blockIdx.x;
     double s[kBatchMax];
 #pragma unroll
     for (int b = 0; b < kBatchMax; b++) s[b] = 0;
-    const double* a = A + (size_t)row * n;
+    const double* a = A + (size_t)row * ld;
     for (int j = threadIdx.x; j < n; j += 64) {
         const double aj = a[j];
 #pragma unroll
@@ -1566,8 +1559,8 @@ void launch_coarsest_batch(const double* Ainv, int n3, const int* rowslot, int n
     if (nrows <= 0) return;
     hipLaunchKernelGGL((k_gather_rows_b<T>), dim3((nrows + 255) / 256), dim3(256), 0, s, rowslot, nrows, F, N, 3 * N,
                        nb, fbuf);
-    hipLaunchKernelGGL((k_dense_gemv_b<T>), dim3(n3), dim3(64), 0, s, Ainv, n3, (const double*)fbuf, rowslot, U, N,
-                       3 * N, nb);
+    hipLaunchKernelGGL((k_dense_gemv_b<T>), dim3(n3), dim3(64), 0, s, Ainv, n3, dense_ld(n3), (const double*)fbuf,
+                       rowslot, U, N, 3 * N, nb);
     RT_HIP(hipGetLastError());
 }
 

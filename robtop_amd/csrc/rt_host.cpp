@@ -15,7 +15,6 @@
 #include "net_internal.h"
 
 #include <rocblas/rocblas.h>
-#include <rocsolver/rocsolver.h>
 
 // dense symmetric eigensolver (defined with the block Lanczos search below)
 static void jacobi_eigen(int n, std::vector<double>& A, std::vector<double>& w, std::vector<double>& V);
@@ -82,6 +81,16 @@ struct Level {
     size_t ne_box() const { return (size_t)e[0] * e[1] * e[2]; }
 };
 
+// what the exact solve of a level needs of its geometry, laid out once (node
+// activity is fixed with the hierarchy): the unknowns' order, their neighbours
+// and the elimination's steps
+struct DirectPlan {
+    int nr = -1;                          // active nodes; -1: not built
+    DBuf nbcol;                           // [27 r + nb] row of the neighbour, -1: none
+    GjPlan steps;
+    std::vector<double> pos;              // node positions in the unknowns' order
+};
+
 struct Hier {
     int R = 0, nlayers = 0;
     std::vector<int> layer_active;
@@ -105,9 +114,10 @@ struct Hier {
     LevelVecs<float> pc32;
     DBuf partials, scal, fbuf, stage;
     int nparts_max = 0;
-    // coarsest: explicit inverse of the dense system (FP64, n3 x n3), factored
-    // with rocSOLVER on the handle's stream
-    DBuf Ainv, rowslot, dinfo;
+    // coarsest: explicit inverse of the dense system (FP64, row stride
+    // dense_ld(n3)), computed on the handle's stream
+    DBuf Ainv, rowslot, dinfo, dwork;
+    DirectPlan dplan, pcdplan;
     rocblas_handle blas = nullptr;
     int n3 = 0;
     DBuf fixce;
@@ -588,7 +598,7 @@ static void prolong_from(Hier& H, int li, Vec3<T> Uf, Vec3<const T> Uc, bool ski
 template <typename T>
 static void coarsest(Hier& H, Vec3<const T> F, Vec3<T> U) {
     if (!H.stencil_ready) throw std::logic_error("update_stencil has not been called");
-    launch_coarsest<T>(H.Ainv.as<double>(), H.n3, H.rowslot.as<int>(), 0, F, U, H.fbuf.as<double>(), H.s);
+    launch_coarsest<T>(H.Ainv.as<double>(), H.n3, H.rowslot.as<int>(), F, U, H.fbuf.as<double>(), H.s);
 }
 
 // whether the preconditioner's last fine sweep yields r . z itself (the
@@ -654,7 +664,7 @@ static void vcycle_core(Hier& H, V3<T>& U0, V3<T>& F0, V3<T>& R0, int pre, int p
     auto cyc = [&](auto&& self, int i) -> void {
         if (i == n - 1) {
             if (early)
-                launch_coarsest<T>(H.pcAinv.as<double>(), H.pcn3, H.pcrowslot.as<int>(), 0, Fv(i), Uv(i),
+                launch_coarsest<T>(H.pcAinv.as<double>(), H.pcn3, H.pcrowslot.as<int>(), Fv(i), Uv(i),
                                    H.pcfbuf.as<double>(), H.s);
             else
                 coarsest<T>(H, Fv(i), Uv(i));
@@ -825,44 +835,61 @@ static int rigid_basis(const std::vector<double>& p, std::vector<double>& R) {
     return k;
 }
 
-// dense exact solve of level li: the matrix assembled on the device from its
-// FP64 stencils, Cholesky and inverse there too (rocSOLVER, FP64); Ainv
-// n3 x n3, rowslot[r] = slot of the level's r-th active node
-static void factor_level(Hier& H, int li, DBuf& Ainv, DBuf& rowslot, DBuf& fbuf, int& n3_out) {
+// the unknowns of level li's exact solve: nodes with the level's longest axis
+// slowest, so that the elimination's reach (a node plane) is shortest
+static void direct_plan(Hier& H, int li, DirectPlan& P, DBuf& rowslot) {
     Level& L = H.lv[li];
-    const size_t N = (size_t)L.g.N;
     const int nx = L.g.n[0], ny = L.g.n[1], nz = L.g.n[2];
-    std::vector<int> slots, rowof(N, -1);
-    std::vector<double> pos;
-    for (int z = 0; z < nz; z++)
-        for (int y = 0; y < ny; y++)
-            for (int x = 0; x < nx; x++)
-                if (L.vact[x + (size_t)nx * (y + (size_t)ny * z)]) {
-                    const int s = oct_p(L.g, x, y, z);
-                    rowof[s] = (int)slots.size();
-                    slots.push_back(s);
-                    pos.push_back(x); pos.push_back(y); pos.push_back(z);
-                }
-    const int nr = (int)slots.size(), n = 3 * nr;
-    std::vector<int> nbcol((size_t)27 * nr, -1);
-    for (int z = 0; z < nz; z++)
-        for (int y = 0; y < ny; y++)
-            for (int x = 0; x < nx; x++) {
-                const int r = rowof[oct_p(L.g, x, y, z)];
-                if (r < 0) continue;
-                for (int nb = 0; nb < 27; nb++) {
-                    const int jx = x + nb % 3 - 1, jy = y + nb / 3 % 3 - 1, jz = z + nb / 9 - 1;
-                    if (jx < 0 || jy < 0 || jz < 0 || jx >= nx || jy >= ny || jz >= nz) continue;
-                    nbcol[(size_t)27 * r + nb] = rowof[oct_p(L.g, jx, jy, jz)];
+    int ax[3] = {0, 1, 2};                // fastest to slowest
+    std::stable_sort(ax, ax + 3, [&](int a, int b) { return L.g.n[a] < L.g.n[b]; });
+    std::vector<int> slots, rowof((size_t)L.g.N, -1), at;
+    P.pos.clear();
+    int i[3];
+    for (i[ax[2]] = 0; i[ax[2]] < L.g.n[ax[2]]; i[ax[2]]++)
+        for (i[ax[1]] = 0; i[ax[1]] < L.g.n[ax[1]]; i[ax[1]]++)
+            for (i[ax[0]] = 0; i[ax[0]] < L.g.n[ax[0]]; i[ax[0]]++) {
+                const int x = i[0], y = i[1], z = i[2];
+                if (!L.vact[x + (size_t)nx * (y + (size_t)ny * z)]) continue;
+                const int s = oct_p(L.g, x, y, z);
+                rowof[s] = (int)slots.size();
+                slots.push_back(s);
+                for (int v : {x, y, z}) {
+                    P.pos.push_back(v);
+                    at.push_back(v);
                 }
             }
+    const int nr = (int)slots.size(), nb64 = dense_ld(3 * nr) / 64;
+    std::vector<int> nbcol((size_t)27 * nr, -1);
+    std::vector<int> reach(nb64, 0);
+    for (int r = 0; r < nr; r++) {
+        int far = r;
+        for (int nb = 0; nb < 27; nb++) {
+            const int jx = at[3 * r] + nb % 3 - 1, jy = at[3 * r + 1] + nb / 3 % 3 - 1, jz = at[3 * r + 2] + nb / 9 - 1;
+            if (jx < 0 || jy < 0 || jz < 0 || jx >= nx || jy >= ny || jz >= nz) continue;
+            const int c = nbcol[(size_t)27 * r + nb] = rowof[oct_p(L.g, jx, jy, jz)];
+            far = std::max(far, c);
+        }
+        for (int d = 3 * r; d < 3 * r + 3; d++) reach[d / 64] = std::max(reach[d / 64], (3 * far + 2) / 64 + 1);
+    }
+    P.steps = spd_inverse_plan(reach);
     rowslot.ensure(sizeof(int) * (size_t)std::max(nr, 1));
-    DBuf nbc;
-    nbc.alloc(sizeof(int) * std::max<size_t>(nbcol.size(), 1));
+    P.nbcol.ensure(sizeof(int) * std::max<size_t>(nbcol.size(), 1));
     RT_HIP(hipMemcpyAsync(rowslot.p, slots.data(), sizeof(int) * (size_t)nr, hipMemcpyHostToDevice, H.s));
-    RT_HIP(hipMemcpyAsync(nbc.p, nbcol.data(), sizeof(int) * nbcol.size(), hipMemcpyHostToDevice, H.s));
-    Ainv.ensure(sizeof(double) * std::max<size_t>((size_t)n * n, 1));
-    launch_dense_from_stencil(L.st64.as<double>(), N, rowslot.as<int>(), nbc.as<int>(), nr, Ainv.as<double>(), H.s);
+    RT_HIP(hipMemcpyAsync(P.nbcol.p, nbcol.data(), sizeof(int) * nbcol.size(), hipMemcpyHostToDevice, H.s));
+    RT_HIP(hipStreamSynchronize(H.s));
+    P.nr = nr;
+}
+
+// dense exact solve of level li: the matrix assembled on the device from its
+// FP64 stencils and inverted there (k_dense.hip); Ainv has row stride
+// dense_ld(n3), rowslot[r] = slot of the level's r-th active node
+static void factor_level(Hier& H, int li, DirectPlan& P, DBuf& Ainv, DBuf& rowslot, DBuf& fbuf, int& n3_out) {
+    Level& L = H.lv[li];
+    const size_t N = (size_t)L.g.N;
+    if (P.nr < 0) direct_plan(H, li, P, rowslot);
+    const int nr = P.nr, n = 3 * nr, ld = dense_ld(n);
+    Ainv.ensure(sizeof(double) * std::max<size_t>((size_t)ld * ld, 1));
+    launch_dense_from_stencil(L.st64.as<double>(), N, rowslot.as<int>(), P.nbcol.as<int>(), nr, Ainv.as<double>(), H.s);
     ensure_blas(H);
     // No supports (the no-support modes): the level's matrix has the rigid
     // motions R of its nodes as null space. The reference's coarsest solve is
@@ -871,40 +898,32 @@ static void factor_level(Hier& H, int li, DBuf& Ainv, DBuf& rowslot, DBuf& fbuf,
     // A + a R R^T is factored and the stored inverse is P (A + a R R^T)^-1 P.
     const bool singular = !has_supports(H);
     DBuf Rd_;
+    GjPlan full;
     if (singular) {
         std::vector<double> R;
-        if (rigid_basis(pos, R) != 6) throw std::domain_error("level has fewer than 6 rigid motions");
+        if (rigid_basis(P.pos, R) != 6) throw std::domain_error("level has fewer than 6 rigid motions");
         Rd_.alloc(sizeof(double) * R.size());
         RT_HIP(hipMemcpyAsync(Rd_.p, R.data(), sizeof(double) * R.size(), hipMemcpyHostToDevice, H.s));
         std::vector<double> diag(n);
-        RT_HIP(hipMemcpy2DAsync(diag.data(), sizeof(double), Ainv.p, sizeof(double) * (size_t)(n + 1), sizeof(double),
+        RT_HIP(hipMemcpy2DAsync(diag.data(), sizeof(double), Ainv.p, sizeof(double) * (size_t)(ld + 1), sizeof(double),
                                 n, hipMemcpyDeviceToHost, H.s));
         RT_HIP(hipStreamSynchronize(H.s));
         double a = 0;
         for (double d : diag) a += d;
         a /= n;
         gemm(H, rocblas_operation_none, rocblas_operation_transpose, n, n, 6, a, Rd_.as<double>(), n,
-             Rd_.as<double>(), n, 1.0, Ainv.as<double>(), n);
+             Rd_.as<double>(), n, 1.0, Ainv.as<double>(), ld);
+        full = spd_inverse_plan(std::vector<int>(ld / 64, ld / 64));   // R R^T couples every unknown
     }
-    // Cholesky and inverse (rocSOLVER, FP64), then mirror the triangle the
-    // inverse was written to so the GEMV can read whole rows
     H.dinfo.ensure(sizeof(int));
-    auto info_ok = [&](const char* what) {
-        int info = 0;
-        RT_HIP(hipMemcpyAsync(&info, H.dinfo.p, sizeof(int), hipMemcpyDeviceToHost, H.s));
-        RT_HIP(hipStreamSynchronize(H.s));
-        if (info != 0)
-            throw std::domain_error(std::string("coarsest system: ") + what + " failed (not positive definite; no supports?)");
-    };
-    if (rocsolver_dpotrf(H.blas, rocblas_fill_lower, n, Ainv.as<double>(), n, H.dinfo.as<int>()) !=
-        rocblas_status_success)
-        throw std::runtime_error("rocsolver_dpotrf failed");
-    info_ok("Cholesky factorisation");
-    if (rocsolver_dpotri(H.blas, rocblas_fill_lower, n, Ainv.as<double>(), n, H.dinfo.as<int>()) !=
-        rocblas_status_success)
-        throw std::runtime_error("rocsolver_dpotri failed");
-    info_ok("inverse");
-    launch_mirror_upper(Ainv.as<double>(), n, H.s);
+    H.dwork.ensure(sizeof(double) * spd_inverse_work(n));
+    launch_spd_inverse(Ainv.as<double>(), n, singular ? full : P.steps, H.dwork.as<double>(),
+                       H.dinfo.as<int>(), H.s);
+    int info = 0;
+    RT_HIP(hipMemcpyAsync(&info, H.dinfo.p, sizeof(int), hipMemcpyDeviceToHost, H.s));
+    RT_HIP(hipStreamSynchronize(H.s));
+    if (info != 0)
+        throw std::domain_error("coarsest system: Cholesky factorisation failed (not positive definite; no supports?)");
     if (singular) {
         // M <- P M P = M - G R^T - R G^T + R (R^T G) R^T, G = M R
         const double* R = Rd_.as<double>();
@@ -913,30 +932,29 @@ static void factor_level(Hier& H, int li, DBuf& Ainv, DBuf& rowslot, DBuf& fbuf,
         T.alloc(sizeof(double) * (size_t)n * 6);
         S.alloc(sizeof(double) * 36);
         double* M = Ainv.as<double>();
-        gemm(H, rocblas_operation_none, rocblas_operation_none, n, 6, n, 1.0, M, n, R, n, 0.0, G.as<double>(), n);
+        gemm(H, rocblas_operation_none, rocblas_operation_none, n, 6, n, 1.0, M, ld, R, n, 0.0, G.as<double>(), n);
         gemm(H, rocblas_operation_transpose, rocblas_operation_none, 6, 6, n, 1.0, R, n, G.as<double>(), n, 0.0,
              S.as<double>(), 6);
         gemm(H, rocblas_operation_none, rocblas_operation_none, n, 6, 6, 1.0, R, n, S.as<double>(), 6, 0.0,
              T.as<double>(), n);
-        gemm(H, rocblas_operation_none, rocblas_operation_transpose, n, n, 6, -1.0, G.as<double>(), n, R, n, 1.0, M, n);
-        gemm(H, rocblas_operation_none, rocblas_operation_transpose, n, n, 6, -1.0, R, n, G.as<double>(), n, 1.0, M, n);
-        gemm(H, rocblas_operation_none, rocblas_operation_transpose, n, n, 6, 1.0, T.as<double>(), n, R, n, 1.0, M, n);
+        gemm(H, rocblas_operation_none, rocblas_operation_transpose, n, n, 6, -1.0, G.as<double>(), n, R, n, 1.0, M, ld);
+        gemm(H, rocblas_operation_none, rocblas_operation_transpose, n, n, 6, -1.0, R, n, G.as<double>(), n, 1.0, M, ld);
+        gemm(H, rocblas_operation_none, rocblas_operation_transpose, n, n, 6, 1.0, T.as<double>(), n, R, n, 1.0, M, ld);
         RT_HIP(hipStreamSynchronize(H.s));
     }
     n3_out = n;
     fbuf.ensure(sizeof(double) * (size_t)std::max(n, 1));
-    RT_HIP(hipStreamSynchronize(H.s));
 }
 
 static void factor_coarsest(Hier& H) {
-    factor_level(H, (int)H.lv.size() - 1, H.Ainv, H.rowslot, H.fbuf, H.n3);
+    factor_level(H, (int)H.lv.size() - 1, H.dplan, H.Ainv, H.rowslot, H.fbuf, H.n3);
     // the preconditioner's cycle stops one level early when that level is
     // small enough to solve exactly (its smoothing passes cost launches, not
     // bandwidth); the reference-semantics V-cycle keeps the whole hierarchy
     const int n = (int)H.lv.size();
     H.pc_levels = n;
     if (n >= 3 && 3 * (long long)H.lv[n - 2].n_vact <= H.pc_direct_dofs) {
-        factor_level(H, n - 2, H.pcAinv, H.pcrowslot, H.pcfbuf, H.pcn3);
+        factor_level(H, n - 2, H.pcdplan, H.pcAinv, H.pcrowslot, H.pcfbuf, H.pcn3);
         H.pc_levels = n - 1;
     }
 }

@@ -173,11 +173,22 @@ template <typename T>
 void launch_prolong(const Geom& gf, const int of[3], Vec3<T> Uf, const uint8_t* vflag_f, const Geom& gc,
                     const int oc[3], Vec3<const T> Uc, int ratio, bool skip_fixed, hipStream_t s);
 template <typename T>
-void launch_coarsest(const double* Ainv, int n3, const int* rowslot, int unused, Vec3<const T> F, Vec3<T> U,
-                     double* fbuf, hipStream_t s);
-void launch_mirror_upper(double* A, int n, hipStream_t s);
+void launch_coarsest(const double* Ainv, int n3, const int* rowslot, Vec3<const T> F, Vec3<T> U, double* fbuf,
+                     hipStream_t s);
 void launch_dense_from_stencil(const double* st, size_t N, const int* slots, const int* nbcol, int nr, double* A,
                                hipStream_t s);
+// k_dense.hip: explicit inverse of a dense SPD system; row stride (and padded
+// order) of the n x n matrices
+inline int dense_ld(int n) { return (n + 63) / 64 * 64; }
+// one 64-row pivot block of the inversion and the 64-row blocks it is combined
+// with, and the blocks of each launch: uncoupled ones together, no row in the
+// range of more than two of them
+constexpr int kGjMax = 4;
+struct GjPivot { int k, lo, hi; };
+typedef std::vector<std::vector<GjPivot>> GjPlan;
+GjPlan spd_inverse_plan(const std::vector<int>& reach);
+size_t spd_inverse_work(int n);
+void launch_spd_inverse(double* A, int n, const GjPlan& plan, double* work, int* info, hipStream_t s);
 // x = sum_i c[i] h[i], k <= 8 FP64 vectors of length n
 void launch_lincomb(double* x, const double* const* h, const double* c, int k, size_t n, hipStream_t s);
 // floating-cluster deflation (k_island.hip): builds the islands of stiff

@@ -1,0 +1,92 @@
+"""The exact solve of the coarsest level (blocked inversion in 64-row pivot
+blocks) against numpy's dense solve of the same stencils, on systems of
+a partly filled last block, with a band so narrow that several blocks
+are eliminated side by side, with the longest axis along each direction, and
+with ragged node planes. The explicit inverse's forward error is bounded by
+n eps cond(A) (n: order; double precision)."""
+import numpy as np
+import pytest
+
+from robtop_amd.workloads import cube_bits
+
+
+def solid(R, ex, ey, ez, holes=False):
+    a = np.zeros((R, R, R), bool)
+    a[:ex, :ey, :ez] = True
+    if holes:
+        a[ex // 4:ex // 3, :, :ez // 2] = False
+        a[ex // 2:, ey // 2:, ez // 2:] = False
+    return a
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("R,ex,ey,ez,holes", [
+    (32, 24, 12, 12, False),       # 112 nodes, 336 unknowns: six blocks, the last one ragged
+    (16, 16, 16, 16, False),       # 125 nodes, 375 unknowns
+    (32, 28, 28, 28, False),       # 512 nodes: the band covers a third of the matrix
+    (256, 256, 8, 8, False),       # 585 nodes in a narrow band: four segments and three separators
+    (128, 8, 8, 128, False),       # the longest axis along z
+    (64, 20, 56, 24, True),        # the longest axis along y, node planes of different sizes
+])
+def test_coarsest_solve_matches_dense_solve(R, ex, ey, ez, holes):
+    import robtop_amd as rt
+    print(f"[dense] {R} {ex}x{ey}x{ez} holes={holes}", flush=True)
+    hg = rt.HierarchyGrid.genFromMesh(cube_bits(solid(R, ex, ey, ez, holes)), R)
+    hg.set_material(1e6, 0.4, 3.0)
+    nx, ny, nz = hg[0].nodes
+    _, vact = hg[0].masks()
+    fixed = np.zeros((nz, ny, nx), bool)
+    fixed[:, :, 0] = vact.reshape(nz, ny, nx)[:, :, 0]
+    hg.set_support(fixed.reshape(-1))
+    rng = np.random.default_rng(R + ex)
+    eact, _ = hg[0].masks()
+    hg.set_density((rng.uniform(0.2, 1.0, eact.size) * eact).astype(np.float32))
+    hg.set_precision(64)
+    hg.update_stencil()
+    g = hg[hg.n_levels - 1]
+    st = g.getStencil()
+    cx, cy, cz = (int(v) for v in g.nodes)
+    _, act = g.masks()
+    idx = -np.ones(act.size, int)
+    idx[act] = np.arange(act.sum())
+    n = 3 * int(act.sum())
+    A = np.zeros((n, n))
+    for v in np.nonzero(act)[0]:
+        x, y, z = v % cx, v // cx % cy, v // (cx * cy)
+        for nb in range(27):
+            jx, jy, jz = x + nb % 3 - 1, y + nb // 3 % 3 - 1, z + nb // 9 - 1
+            if not (0 <= jx < cx and 0 <= jy < cy and 0 <= jz < cz):
+                continue
+            j = idx[jx + cx * (jy + cy * jz)]
+            if j >= 0:
+                A[3 * idx[v]:3 * idx[v] + 3, 3 * j:3 * j + 3] = st[nb, :, v].reshape(3, 3)
+    f = np.zeros((3, act.size))
+    f[:, act] = rng.standard_normal((3, int(act.sum())))
+    g.setForce(f)
+    g.setDisplacement(np.zeros_like(f))
+    g.solve_fem_host()
+    u = g.getDisplacement()[:, act].T.reshape(-1)
+    ref = np.linalg.solve(A, f[:, act].T.reshape(-1))
+    bound = n * np.finfo(float).eps * np.linalg.cond(A)
+    err = np.linalg.norm(u - ref) / np.linalg.norm(ref)
+    print(f"n {n}, error {err:.2e}, bound {bound:.2e}", flush=True)
+    assert err <= bound
+    hg.close()
+
+
+@pytest.mark.gpu
+def test_zero_stiffness_is_refused():
+    """A zero stiffness off the supports: the first pivot is not positive, which is reported, not solved."""
+    import robtop_amd as rt
+    hg = rt.HierarchyGrid.genFromMesh(cube_bits(solid(16, 16, 16, 16)), 16)
+    hg.set_material(1e6, 0.4, 3.0)
+    nx, ny, nz = hg[0].nodes
+    _, vact = hg[0].masks()
+    fixed = np.zeros((nz, ny, nx), bool)
+    fixed[:, :, 0] = vact.reshape(nz, ny, nx)[:, :, 0]
+    hg.set_support(fixed.reshape(-1))
+    hg.set_density(np.zeros(hg[0].n_elements_box, np.float32))   # every stiffness 0: every pivot 0
+    print("[dense] zero stiffness", flush=True)
+    with pytest.raises(rt.RobtopError, match="not positive definite"):
+        hg.update_stencil()
+    hg.close()
