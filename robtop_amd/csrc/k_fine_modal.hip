@@ -27,7 +27,7 @@ namespace rt {
 #ifndef RT_MODAL_TX
 #define RT_MODAL_TX 31
 #endif
-// z planes per workgroup (Geom::zc, default 24, chosen per hierarchy by the
+// z planes per workgroup (Geom::zc, picked from the box (pick_zc) or by the
 // autotuner). Measured at 511 x 256 x 256 (ms per residual): 8 planes 0.81,
 // 12 0.80, 16 0.81, 24 0.79, 32 0.86, 64 1.07; a 15 x 15 node tile instead of
 // 31 x 7: 0.95.

@@ -76,6 +76,7 @@ struct Level {
     DBuf st64, st32, KEc;
     DBuf st16;                            // bfloat16 copy for FP32 preconditioner cycles (optional)
     DBuf tile_act;                        // finest level: mask of residual / apply tiles holding an active node
+    std::vector<uint8_t> col_act;         // the same per tile column and node plane
     BVec<float> bU, bF, bR;               // batched preconditioner cycle (worst-case block solves)
     size_t nn_box() const { return (size_t)g.n[0] * g.n[1] * g.n[2]; }
     size_t ne_box() const { return (size_t)e[0] * e[1] * e[2]; }
@@ -435,24 +436,62 @@ static void ensure_partials(Hier& H) {
     H.scal.alloc(sizeof(double) * 16);
 }
 
+// node planes of the residual / apply kernels' tile columns that hold an
+// active node: col_act[z * columns + column]
+static void build_column_act(Level& L) {
+    int tx, ty;
+    modal_tile_dims(&tx, &ty);
+    const int nx = L.g.n[0], ny = L.g.n[1], nz = L.g.n[2];
+    const int gx = (nx + tx - 1) / tx, gy = (ny + ty - 1) / ty;
+    L.col_act.assign((size_t)gx * gy * nz, 0);
+    for (int z = 0; z < nz; z++)
+        for (int y = 0; y < ny; y++) {
+            const uint8_t* row = L.vact.data() + (size_t)nx * ((size_t)y + (size_t)ny * z);
+            uint8_t* m = L.col_act.data() + (size_t)gx * ((size_t)(y / ty) + (size_t)gy * z);
+            for (int x = 0; x < nx; x++) m[x / tx] |= row[x];
+        }
+}
+
+// the column activity of chunks of zc planes (Geom::tile_act's layout)
+static std::vector<uint8_t> tile_mask(const Level& L, int zc) {
+    const int nz = L.g.n[2], cols = (int)(L.col_act.size() / nz), gz = (nz + zc - 1) / zc;
+    std::vector<uint8_t> m((size_t)cols * gz, 0);
+    for (int z = 0; z < nz; z++)
+        for (int c = 0; c < cols; c++) m[(size_t)(z / zc) * cols + c] |= L.col_act[(size_t)z * cols + c];
+    return m;
+}
+
 // Finest-level work mask (Geom::tile_act) from the active nodes: the residual /
 // apply kernels skip tiles that hold no active node (their outputs are absent
 // slots, never written). Rebuilt whenever Geom::zc changes.
 static void build_tile_mask(Level& L) {
-    int tx, ty;
-    modal_tile_dims(&tx, &ty);
-    const int nx = L.g.n[0], ny = L.g.n[1], nz = L.g.n[2], tz = L.g.zc;
-    const int gx = (nx + tx - 1) / tx, gy = (ny + ty - 1) / ty, gz = (nz + tz - 1) / tz;
-    std::vector<uint8_t> m((size_t)gx * gy * gz, 0);
-    for (int z = 0; z < nz; z++)
-        for (int y = 0; y < ny; y++) {
-            const uint8_t* row = L.vact.data() + (size_t)nx * ((size_t)y + (size_t)ny * z);
-            for (int x = 0; x < nx; x++)
-                if (row[x]) m[(size_t)(x / tx) + (size_t)gx * ((size_t)(y / ty) + (size_t)gy * (z / tz))] = 1;
-        }
+    const std::vector<uint8_t> m = tile_mask(L, L.g.zc);
     L.tile_act.alloc(m.size());
     RT_HIP(hipMemcpy(L.tile_act.p, m.data(), m.size(), hipMemcpyHostToDevice));
     L.g.tile_act = L.tile_act.as<uint8_t>();
+}
+
+// z planes per residual / apply workgroup. A workgroup takes zc + 1 steps of
+// about the same length, and 1024 of them are resident (four per CU), so the
+// kernel's time goes as rounds x (zc + 1): long columns where the box fills the
+// chip anyway, down to single planes where it does not. Measured (FP32
+// residual, us) at zc = 24 and at the zc this picks: 48 x 24 x 24 elements 42.6
+// and 6.3 (1), 64 x 32 x 32 65.9 and 7.1 (1), 128 x 64 x 64 44.9 and 19.2 (4),
+// 256 x 128 x 128 106.7 and 85.4 (12), 384 x 192 x 192 291 and 274 (8); 160^3
+// and 511 x 256 x 256 stay at 24.
+static int pick_zc(const Level& L) {
+    int best = 24;
+    long long least = -1;
+    for (int zc : {24, 16, 12, 8, 6, 4, 3, 2, 1}) {
+        long long tiles = 0;
+        for (uint8_t m : tile_mask(L, zc)) tiles += m;
+        const long long cost = (tiles + 1023) / 1024 * (zc + 1);
+        if (least < 0 || cost < least) {
+            least = cost;
+            best = zc;
+        }
+    }
+    return best;
 }
 
 static void setup_device(Hier& H) {
@@ -478,6 +517,8 @@ static void setup_device(Hier& H) {
         if (L.scale / H.lv[li - 1].scale == 4)
             H.xfer.ensure(sizeof(double) * restrict_scratch_elems(H.lv[li - 1].g, L.g));
     }
+    build_column_act(L0);
+    L0.g.zc = pick_zc(L0);
     ensure_partials(H);
     build_tile_mask(L0);
 }
