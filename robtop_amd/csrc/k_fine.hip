@@ -20,6 +20,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include <utility>
 
 namespace rt {
@@ -172,6 +173,11 @@ __device__ __forceinline__ void nb_row(const Geom& g, int vb, const KeC<T>& K, c
     nb_step<T, C, CHECK_FIX, NBM + 1, Z0>(g, vb, K, B, acc);   // skips the node itself
 }
 
+// the neighbour rows in the order of every smoother kernel here: the node's
+// own row last, since the row kernel has its second node's neighbours there
+// only once the first ones are relaxed
+typedef std::integer_sequence<int, 0, 1, 2, 3, 5, 6, 7, 8, 4> RowOrder;
+
 template <typename T, int C, bool CHECK_FIX, bool Z0, int... ROWs>
 __device__ __forceinline__ void nb_all(const Geom& g, int vb, const KeC<T>& K, const GsBufs& B, T (&acc)[8][3],
                                        std::integer_sequence<int, ROWs...>) {
@@ -210,7 +216,7 @@ __device__ __forceinline__ void gs_node(const Geom& g, int base, const KeC<T>& K
     T acc[8][3];
 #pragma unroll
     for (int w = 0; w < 8; w++) acc[w][0] = acc[w][1] = acc[w][2] = T(0);
-    nb_all<T, C, CHECK_FIX, Z0>(g, vb, K, B, acc, std::make_integer_sequence<int, 9>{});
+    nb_all<T, C, CHECK_FIX, Z0>(g, vb, K, B, acc, RowOrder{});
     KU[0] = KU[1] = KU[2] = T(0);
 #pragma unroll
     for (int i = 0; i < 9; i++) S[i] = T(0);
@@ -308,17 +314,6 @@ __device__ __forceinline__ double gs_blk_sum(double v) {
     return t;
 }
 
-// rows relaxed one after another by each workgroup of the smoother (rows of one
-// launch never neighbour each other). Measured at 511 x 256 x 256 elements: one
-// row per workgroup 1.06 ms per sweep, two 1.13 ms, four 1.24 ms. Taking the
-// rows of a launch in compact (y, z) tiles (4x32 to 64x4 rows) instead of
-// y-fastest order changed the sweep by less than 1 %, and loading both
-// phases' node flags before the first phase (so no phase waits on its flag)
-// changed a launch by 0.1 %.
-#ifndef RT_GS_ROWS
-#define RT_GS_ROWS 1
-#endif
-
 // optional occupancy target (waves per SIMD) for the smoother, a build-time knob
 #if defined(RT_GS_WAVES_PER_EU) && RT_GS_WAVES_PER_EU > 0
 #define RT_GS_ATTR __attribute__((amdgpu_waves_per_eu(RT_GS_WAVES_PER_EU)))
@@ -337,18 +332,323 @@ __global__ void __launch_bounds__(256) RT_GS_ATTR k_fine_gs_pair(Geom g, Vec3<T>
     double fu = 0;
     double* fup = DOT ? &fu : nullptr;
     const int nhy = (g.n[1] - CY + 1) >> 1;
-    const int first = xcd_row(blockIdx.x, gridDim.x) * RT_GS_ROWS;
+    const int row = xcd_row(blockIdx.x, nrows);
     const int nbytes = g.N * (int)sizeof(T);
     const GsBufs B = {rsrc(U.c[0], nbytes), rsrc(U.c[1], nbytes), rsrc(U.c[2], nbytes), rsrc(rhop, g.N * 4),
                       rsrc(vflag, g.N)};
     constexpr int CA = (REV ? 1 : 0) | (CY << 1) | (CZ << 2);
-    for (int r = 0; r < RT_GS_ROWS; r++) {
-        const int row = first + r;   // uniform across the workgroup
-        if (row >= nrows) break;
-        const int j = row % nhy, k = row / nhy;
-        gs_row_phase<T, CA, ZS, Z0>(g, j, k, U, F, vflag, K, B, REV, fup);
-        __syncthreads();
-        gs_row_phase<T, CA ^ 1, ZS, Z0>(g, j, k, U, F, vflag, K, B, REV, fup);
+    const int j = row % nhy, k = row / nhy;
+    gs_row_phase<T, CA, ZS, Z0>(g, j, k, U, F, vflag, K, B, REV, fup);
+    __syncthreads();
+    gs_row_phase<T, CA ^ 1, ZS, Z0>(g, j, k, U, F, vflag, K, B, REV, fup);
+    if constexpr (DOT) {
+        const double t = gs_blk_sum(fu);
+        if (threadIdx.x == 0) fu_part[blockIdx.x] = t;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// The row kernel: k_fine_gs_pair's launch with both x parities of a thread's
+// place in the row at once. A thread holds the nodes x = 2 i and 2 i + 1: of
+// every other row they need the same four values per component, E(2i), E(2i+2)
+// and O(2i-1), O(2i+1) (consecutive slots: two two-wide loads), and of the
+// elements three values for four. All of that is read-only during the launch,
+// so it is loaded and multiplied once, before the first parity is relaxed;
+// only the own row's new values have to cross the barrier, through LDS.
+//
+// Against a pass per parity it issues 2 loads where that issued 4, reads the
+// neighbour rows from the caches once instead of twice, and waits for memory
+// once. Same arithmetic per node and the same order, so the same bits.
+//
+// Bound: FP32 FMA issue (0.55 ms of a sweep at 511 x 256 x 256 elements) with
+// the latency of the row loads, which 4 waves per SIMD hide in part; the pass
+// per parity was bound by its reads from beyond L2, 1.48 GB a launch against
+// 0.89 now. Measured, ms per FP32 sweep: 511 x 256 x 256 1.03 -> 0.79, 256 x
+// 128 x 128 0.156 -> 0.130, 128 x 64 x 64 0.041 -> 0.037; FP64 1.66 -> 1.20,
+// 0.195 -> 0.178, 0.049 -> 0.045. A spilled register or a fifth wave of one
+// lane (see row_shape) costs all of that: 5 waves per SIMD with 7 spilled
+// registers 1.23, a workgroup of 257 threads 0.96.
+// ---------------------------------------------------------------------------
+// a point that no load and no term of the sums moves across (the sums pass
+// through it; it emits nothing)
+template <typename T>
+__device__ __forceinline__ void row_fence(T (&aE)[8][3], T (&aO)[8][3]) {
+#pragma unroll
+    for (int w = 0; w < 8; w++)
+        asm volatile("" : "+v"(aE[w][0]), "+v"(aE[w][1]), "+v"(aE[w][2]), "+v"(aO[w][0]), "+v"(aO[w][1]), "+v"(aO[w][2])
+                     : : "memory");
+}
+
+template <typename T> struct RowVals {
+    Two<T> e[3], o[3];
+    uint8_t fl[4];          // CHECK_FIX: flags of e.lo, e.hi, o.lo, o.hi
+};
+
+// whether the rows (DY, DZ) still hold 0 in a zero-start sweep (both colours of
+// a row come later than both of the pair, or neither)
+template <int CE, int ROW, bool Z0>
+constexpr bool row_used() { return !(Z0 && nb_colour<CE, 0, ROW % 3 - 1, ROW / 3 - 1>() > CE); }
+
+template <typename T, int CE, bool CHECK_FIX, int ROW, bool Z0>
+__device__ __forceinline__ void row_load(const Geom& g, int vb, const GsBufs& B, RowVals<T>& v) {
+    if constexpr (row_used<CE, ROW, Z0>()) {
+        constexpr int DY = ROW % 3 - 1, DZ = ROW / 3 - 1;
+        const int vo = vb * (int)sizeof(T);
+        const int se = rel_off<CE, 0, DY, DZ>(g), so = rel_off<CE, -1, DY, DZ>(g);
+        const __amdgpu_buffer_rsrc_t u[3] = {B.u0, B.u1, B.u2};
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            v.e[c] = bload2<T>(u[c], vo, se * (int)sizeof(T));
+            v.o[c] = bload2<T>(u[c], vo, so * (int)sizeof(T));
+        }
+        if constexpr (CHECK_FIX) {
+            v.fl[0] = bload_u8(B.flag, vb, se); v.fl[1] = bload_u8(B.flag, vb, se + 1);
+            v.fl[2] = bload_u8(B.flag, vb, so); v.fl[3] = bload_u8(B.flag, vb, so + 1);
+        }
+    }
+}
+
+template <typename T, int CE, bool CHECK_FIX, int ROW, bool Z0>
+__device__ __forceinline__ void row_use(const KeC<T>& K, RowVals<T>& v, T (&aE)[8][3], T (&aO)[8][3]) {
+    if constexpr (row_used<CE, ROW, Z0>()) {
+        constexpr int NBM = 9 * (ROW / 3) + 3 * (ROW % 3);   // dx = -1; dx = 0, +1 follow
+        if constexpr (CHECK_FIX) {
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                if (v.fl[0] & NF_FIXED) v.e[c].lo = T(0);
+                if (v.fl[1] & NF_FIXED) v.e[c].hi = T(0);
+                if (v.fl[2] & NF_FIXED) v.o[c].lo = T(0);
+                if (v.fl[3] & NF_FIXED) v.o[c].hi = T(0);
+            }
+        }
+        const auto ws = std::make_integer_sequence<int, 8>{};
+        nb_elems<T, NBM>(aE, K, v.o[0].lo, v.o[1].lo, v.o[2].lo, ws);
+        nb_elems<T, NBM + 2>(aE, K, v.o[0].hi, v.o[1].hi, v.o[2].hi, ws);
+        nb_elems<T, NBM + 1>(aE, K, v.e[0].lo, v.e[1].lo, v.e[2].lo, ws);
+        nb_elems<T, NBM>(aO, K, v.e[0].lo, v.e[1].lo, v.e[2].lo, ws);
+        nb_elems<T, NBM + 2>(aO, K, v.e[0].hi, v.e[1].hi, v.e[2].hi, ws);
+        nb_elems<T, NBM + 1>(aO, K, v.o[0].hi, v.o[1].hi, v.o[2].hi, ws);
+    }
+}
+
+// the eight rows besides the own one, in RowOrder: the values of a row are
+// loaded kRowAhead rows before they are multiplied (the fences keep it at
+// that: the compiler would otherwise start all of them at once and spill), and
+// `last` issues the loads that the node updates need before the last row
+template <typename T> constexpr int kRowAhead = sizeof(T) == 4 ? 1 : 2;
+constexpr int row_at(int i) { return i < 4 ? i : i + 1; }
+
+template <typename T, int CE, bool CHECK_FIX, bool Z0, int I, typename L>
+__device__ __forceinline__ void pair_rows(const Geom& g, int vb, const KeC<T>& K, const GsBufs& B,
+                                          RowVals<T> (&v)[kRowAhead<T> + 1], T (&aE)[8][3], T (&aO)[8][3], L&& last) {
+    if constexpr (I + kRowAhead<T> < 8)
+        row_load<T, CE, CHECK_FIX, row_at(I + kRowAhead<T>), Z0>(g, vb, B, v[(I + kRowAhead<T>) % (kRowAhead<T> + 1)]);
+    if constexpr (I == 7) last();
+    row_fence(aE, aO);
+    row_use<T, CE, CHECK_FIX, row_at(I), Z0>(K, v[I % (kRowAhead<T> + 1)], aE, aO);
+    if constexpr (I < 7) {
+        row_fence(aE, aO);
+        pair_rows<T, CE, CHECK_FIX, Z0, I + 1>(g, vb, K, B, v, aE, aO, last);
+    }
+}
+
+// the old values of the own row's neighbours of the parity relaxed first (REV:
+// the odd node), added to its sums
+template <typename T, int CE, bool CHECK_FIX, bool REV>
+__device__ __forceinline__ void own_load(const Geom& g, int vb, const GsBufs& B, RowVals<T>& v) {
+    const int vo = vb * (int)sizeof(T);
+    const int s = REV ? rel_off<CE, 0, 0, 0>(g) : rel_off<CE, -1, 0, 0>(g), sb = s * (int)sizeof(T);
+    v.e[0] = bload2<T>(B.u0, vo, sb);
+    v.e[1] = bload2<T>(B.u1, vo, sb);
+    v.e[2] = bload2<T>(B.u2, vo, sb);
+    if constexpr (CHECK_FIX) {
+        v.fl[0] = bload_u8(B.flag, vb, s); v.fl[1] = bload_u8(B.flag, vb, s + 1);
+    }
+}
+template <typename T, bool CHECK_FIX>
+__device__ __forceinline__ void own_use(const KeC<T>& K, RowVals<T>& v, T (&a)[8][3]) {
+    if constexpr (CHECK_FIX) {
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            if (v.fl[0] & NF_FIXED) v.e[c].lo = T(0);
+            if (v.fl[1] & NF_FIXED) v.e[c].hi = T(0);
+        }
+    }
+    nb_elems<T, 12>(a, K, v.e[0].lo, v.e[1].lo, v.e[2].lo, std::make_integer_sequence<int, 8>{});
+    nb_elems<T, 14>(a, K, v.e[0].hi, v.e[1].hi, v.e[2].hi, std::make_integer_sequence<int, 8>{});
+}
+
+template <typename T, int W>
+__device__ __forceinline__ void pair_elem(const KeC<T>& K, T pen, const T (&acc)[8][3], T (&KU)[3], T (&S)[9]) {
+    constexpr int vi = 7 - W;
+    KU[0] += pen * acc[W][0];
+    KU[1] += pen * acc[W][1];
+    KU[2] += pen * acc[W][2];
+    S[0] += pen * kc<ke_code_at((3 * vi + 0) * 24 + 3 * vi + 0)>(K);
+    S[1] += pen * kc<ke_code_at((3 * vi + 0) * 24 + 3 * vi + 1)>(K);
+    S[2] += pen * kc<ke_code_at((3 * vi + 0) * 24 + 3 * vi + 2)>(K);
+    S[3] += pen * kc<ke_code_at((3 * vi + 1) * 24 + 3 * vi + 0)>(K);
+    S[4] += pen * kc<ke_code_at((3 * vi + 1) * 24 + 3 * vi + 1)>(K);
+    S[5] += pen * kc<ke_code_at((3 * vi + 1) * 24 + 3 * vi + 2)>(K);
+    S[6] += pen * kc<ke_code_at((3 * vi + 2) * 24 + 3 * vi + 0)>(K);
+    S[7] += pen * kc<ke_code_at((3 * vi + 2) * 24 + 3 * vi + 1)>(K);
+    S[8] += pen * kc<ke_code_at((3 * vi + 2) * 24 + 3 * vi + 2)>(K);
+}
+template <typename T, int... Ws>
+__device__ __forceinline__ void pair_elems(const KeC<T>& K, const float (&pen)[8], const T (&acc)[8][3], T (&KU)[3],
+                                           T (&S)[9], std::integer_sequence<int, Ws...>) {
+    (pair_elem<T, Ws>(K, (T)pen[Ws], acc, KU, S), ...);
+}
+
+// the update of gs_update from the sums; u: the node's old value in, its new one out
+template <typename T, bool REV>
+__device__ __forceinline__ void pair_relax(uint8_t fl, const T (&f)[3], const KeC<T>& K, const float (&pen)[8],
+                                           const T (&acc)[8][3], T (&u)[3]) {
+    if (fl & NF_FIXED) {
+        const T ne = (T)(fl >> 4);
+        u[0] = f[0] / ne; u[1] = f[1] / ne; u[2] = f[2] / ne;
+        return;
+    }
+    T KU[3] = {T(0), T(0), T(0)}, S[9];
+#pragma unroll
+    for (int i = 0; i < 9; i++) S[i] = T(0);
+    pair_elems<T>(K, pen, acc, KU, S, std::make_integer_sequence<int, 8>{});
+    if (!REV) {
+        u[0] = gs_div<T>(f[0] - S[1] * u[1] - S[2] * u[2] - KU[0], S[0]);
+        u[1] = gs_div<T>(f[1] - S[3] * u[0] - S[5] * u[2] - KU[1], S[4]);
+        u[2] = gs_div<T>(f[2] - S[6] * u[0] - S[7] * u[1] - KU[2], S[8]);
+    } else {
+        u[2] = gs_div<T>(f[2] - S[6] * u[0] - S[7] * u[1] - KU[2], S[8]);
+        u[1] = gs_div<T>(f[1] - S[3] * u[0] - S[5] * u[2] - KU[1], S[4]);
+        u[0] = gs_div<T>(f[0] - S[1] * u[1] - S[2] * u[2] - KU[0], S[0]);
+    }
+}
+
+// threads of the row kernel's largest workgroup, and the waves per SIMD that
+// its registers (a pair has 48 sums) are kept down to
+constexpr int kRowThreads = 512;
+template <typename T> constexpr int kRowWaves = sizeof(T) == 4 ? 4 : 2;
+
+template <typename T, int CY, int CZ, bool REV, bool ZS, bool Z0 = false, bool DOT = false>
+__global__ void __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(kRowWaves<T>)))
+k_fine_gs_row(Geom g, Vec3<T> U, Vec3<const T> F, const float* __restrict__ rhop, const uint8_t* __restrict__ vflag,
+              KeC<T> K, int nrows, int rpw, int npr, double* __restrict__ fu_part) {
+    static_assert(!(Z0 && REV), "a zero-start sweep runs forward");
+    constexpr int CE = (CY << 1) | (CZ << 2);
+    __shared__ T sh[3][kRowThreads];         // new values of the parity relaxed first
+    const int nhy = (g.n[1] - CY + 1) >> 1;
+    // thread t: pair i of the workgroup's row r; the last pair's thread also
+    // relaxes the row's last even node where that has no thread (row_shape)
+    const int t = threadIdx.x, r = t / npr, i = t - r * npr;
+    const int row = xcd_row(blockIdx.x, gridDim.x) * rpw + r;
+    const bool in = r < rpw && row < nrows;
+    const int j = in ? row % nhy : 0, k = in ? row / nhy : 0;
+    const int nbytes = g.N * (int)sizeof(T);
+    const GsBufs B = {rsrc(U.c[0], nbytes), rsrc(U.c[1], nbytes), rsrc(U.c[2], nbytes), rsrc(rhop, g.N * 4),
+                      rsrc(vflag, g.N)};
+    const int base = ((k + 1) * g.h[1] + (j + 1)) * g.h[0] + 1 + i;
+    const int vb = base - g.h[0] * g.h[1] - g.h[0] - 1;
+    const int vE = CE * g.cs + base, vO = vE + g.cs;
+    const bool inO = in && 2 * i + 1 < g.n[0], extra = in && i == npr - 1 && 2 * npr < g.n[0];
+    const uint8_t flE = in ? vflag[vE] : 0, flO = inO ? vflag[vO] : 0;
+    T aE[8][3], aO[8][3], fE[3], fO[3], uE[3], uO[3];
+    float pE[8], pO[8];
+    double fu = 0;
+    auto store = [&](int v, const T (&f)[3], const T (&u)[3]) __attribute__((always_inline)) {
+        U.c[0][v] = u[0]; U.c[1][v] = u[1]; U.c[2][v] = u[2];
+        if constexpr (DOT) fu += ((double)f[0] * (double)u[0] + (double)f[1] * (double)u[1]) + (double)f[2] * (double)u[2];
+    };
+    T first[3] = {T(0), T(0), T(0)}, beyond[3] = {T(0), T(0), T(0)};
+    if (!REV && extra) {
+        gs_update<T, CE, ZS, Z0>(g, base + 1, U, F, vflag, K, B, REV, DOT ? &fu : nullptr);
+        if (ZS || !(vflag[vE + 1] & NF_FIXED)) {
+            beyond[0] = U.c[0][vE + 1]; beyond[1] = U.c[1][vE + 1]; beyond[2] = U.c[2][vE + 1];
+        }
+    }
+    // the first rows are on their way before the flags are looked at
+    RowVals<T> v[kRowAhead<T> + 1];
+    auto load_first = [&](auto check) __attribute__((always_inline)) {
+        constexpr bool CHECK = decltype(check)::value;
+        row_load<T, CE, CHECK, 0, Z0>(g, vb, B, v[0]);
+        if constexpr (kRowAhead<T> > 1) row_load<T, CE, CHECK, 1, Z0>(g, vb, B, v[1]);
+    };
+    if (in) load_first(std::false_type{});
+    asm volatile("" ::: "memory");
+    const bool actE = flE & NF_ACTIVE, actO = flO & NF_ACTIVE;
+    if (actE || actO) {
+        // rho^p: the even node's elements are O(i), E(i + 1), the odd one's E(i + 1), O(i + 1)
+        auto pens = [&](auto r) __attribute__((always_inline)) {
+            constexpr int EY = (decltype(r)::value & 1) - 1, EZ = (decltype(r)::value >> 1) - 1;
+            constexpr int w = 2 * (EY + 1) + 4 * (EZ + 1);
+            const Two<float> o = bload2<float>(B.rho, vb * 4, rel_off<CE, -1, EY, EZ>(g) * 4);
+            const float e = bload<float>(B.rho, vb * 4, rel_off<CE, 0, EY, EZ>(g) * 4);
+            pE[w] = o.lo; pE[w + 1] = e; pO[w] = e; pO[w + 1] = o.hi;
+        };
+        auto node_values = [&]() __attribute__((always_inline)) {
+            pens(std::integral_constant<int, 0>{});
+            pens(std::integral_constant<int, 1>{});
+            pens(std::integral_constant<int, 2>{});
+            pens(std::integral_constant<int, 3>{});
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                fE[c] = F.c[c][vE]; fO[c] = F.c[c][vO];
+                uE[c] = Z0 ? T(0) : U.c[c][vE]; uO[c] = Z0 ? T(0) : U.c[c][vO];
+            }
+        };
+        auto sums = [&](auto check) __attribute__((always_inline)) {
+            constexpr bool CHECK = decltype(check)::value;
+            RowVals<T> own;
+            if constexpr (CHECK) load_first(check);
+#pragma unroll
+            for (int w = 0; w < 8; w++)
+#pragma unroll
+                for (int c = 0; c < 3; c++) aE[w][c] = aO[w][c] = T(0);
+            pair_rows<T, CE, CHECK, Z0, 0>(g, vb, K, B, v, aE, aO, [&]() __attribute__((always_inline)) {
+                if constexpr (!Z0) own_load<T, CE, CHECK, REV>(g, vb, B, own);
+                node_values();
+            });
+            if constexpr (!Z0) own_use<T, CHECK>(K, own, REV ? aO : aE);
+        };
+        if (!ZS && ((flE | flO) & NF_NEARFIX)) sums(std::true_type{});
+        else sums(std::false_type{});
+        if constexpr (REV) {
+            pair_relax<T, REV>(flO, fO, K, pO, aO, uO);
+            if (actO) store(vO, fO, uO);
+        } else {
+            pair_relax<T, REV>(flE, fE, K, pE, aE, uE);
+            if (actE) store(vE, fE, uE);
+        }
+        // a support counts as 0 for its neighbours
+        const uint8_t fl = REV ? flO : flE;
+        const bool live = (fl & NF_ACTIVE) && (ZS || !(fl & NF_FIXED));
+#pragma unroll
+        for (int c = 0; c < 3; c++) first[c] = live ? (REV ? uO[c] : uE[c]) : T(0);
+    }
+#pragma unroll
+    for (int c = 0; c < 3; c++) sh[c][t] = first[c];
+    __syncthreads();
+    if (REV ? actE : actO) {
+        T (&a)[8][3] = REV ? aE : aO;
+        // the neighbour pair's value; past the row's ends the extra node's, or the ghost slots' 0
+        const bool end = REV ? i == 0 : i == npr - 1;
+        const int to = end ? t : REV ? t - 1 : t + 1;
+        const T other[3] = {end ? beyond[0] : sh[0][to], end ? beyond[1] : sh[1][to], end ? beyond[2] : sh[2][to]};
+        const T l[3] = {REV ? other[0] : first[0], REV ? other[1] : first[1], REV ? other[2] : first[2]};
+        const T rr[3] = {REV ? first[0] : other[0], REV ? first[1] : other[1], REV ? first[2] : other[2]};
+        nb_elems<T, 12>(a, K, l[0], l[1], l[2], std::make_integer_sequence<int, 8>{});
+        nb_elems<T, 14>(a, K, rr[0], rr[1], rr[2], std::make_integer_sequence<int, 8>{});
+        if constexpr (REV) {
+            pair_relax<T, REV>(flE, fE, K, pE, aE, uE);
+            store(vE, fE, uE);
+        } else {
+            pair_relax<T, REV>(flO, fO, K, pO, aO, uO);
+            store(vO, fO, uO);
+        }
+    }
+    if (REV && extra) gs_update<T, CE, ZS, Z0>(g, base + 1, U, F, vflag, K, B, REV, DOT ? &fu : nullptr);
+    if constexpr (Z0) {   // what a cleared vector would hold
+        if (!actE && in) { U.c[0][vE] = T(0); U.c[1][vE] = T(0); U.c[2][vE] = T(0); }
+        if (!actO && inO) { U.c[0][vO] = T(0); U.c[1][vO] = T(0); U.c[2][vO] = T(0); }
     }
     if constexpr (DOT) {
         const double t = gs_blk_sum(fu);
@@ -447,7 +747,7 @@ __device__ __forceinline__ void gs_node2(const Geom& g, int base, const KeC<T>& 
     T acc[8][3];
 #pragma unroll
     for (int w = 0; w < 8; w++) acc[w][0] = acc[w][1] = acc[w][2] = T(0);
-    nb_all2<T, C, CHECK_FIX, FIRST, REV>(g, vb, K, B, acc, std::make_integer_sequence<int, 9>{});
+    nb_all2<T, C, CHECK_FIX, FIRST, REV>(g, vb, K, B, acc, RowOrder{});
     KU[0] = KU[1] = KU[2] = T(0);
 #pragma unroll
     for (int i = 0; i < 9; i++) S[i] = T(0);
@@ -577,6 +877,36 @@ template void launch_fine_gs_sweep2<float>(const Geom&, Vec3<const float>, Vec3<
 template void launch_fine_gs_sweep2<double>(const Geom&, Vec3<const double>, Vec3<double>, Vec3<const double>,
                                             const float*, const uint8_t*, bool, bool, hipStream_t);
 
+// the row kernel's workgroup for a launch of `rows` rows: rpw whole rows (0: too
+// long for it) of npr pairs in nt threads. Boxes are a multiple of the coarsest
+// spacing plus one node long, so a row's pairs often pass a multiple of 64 by
+// one. Where a launch fills the chip, the last pair's thread then takes the
+// even node left over as well (a wave of one lane would hold a fifth to a half
+// of the wave slots); where it does not, that would only lengthen the chain
+// (128 x 64 x 64 elements: 42.7 against 36.5 us a sweep). Other lengths put
+// several rows into a workgroup if that fills its lanes better and enough
+// workgroups remain.
+struct RowShape { int rpw, nt, npr; };
+template <typename T>
+static RowShape row_shape(const Geom& g, long long rows) {
+    const int nxe = (g.n[0] + 1) / 2;
+    if (nxe > 1 && nxe % 64 == 1 && nxe - 1 <= kRowThreads && rows * (nxe / 64 + 1) > 4096)
+        return RowShape{1, nxe - 1, nxe - 1};
+    RowShape best{0, 0, nxe};
+    double eff = 0;
+    for (int rpw = 1; rpw <= 8 && rpw * nxe <= kRowThreads; rpw++) {
+        if (rpw > 1 && rows / rpw < 1024) break;
+        const int nt = (rpw * nxe + 63) / 64 * 64;
+        const double e = (double)(rpw * nxe) / nt;
+        if (e > eff * 1.05) {
+            eff = e;
+            best.rpw = rpw;
+            best.nt = nt;
+        }
+    }
+    return best;
+}
+
 // pair p = 0..3 relaxes colours (2p, 2p+1), or (2p+1, 2p) when reverse
 // zero_start: the first forward sweep from u = 0 (with zero supports); U may
 // hold anything on entry, and every slot the sweep visits is written
@@ -584,7 +914,9 @@ template void launch_fine_gs_sweep2<double>(const Geom&, Vec3<const double>, Vec
 int fine_gs_pair_blocks(const Geom& g, int pair) {
     const int cy = pair & 1, cz = pair >> 1;
     const long long rows = (long long)((g.n[1] - cy + 1) >> 1) * ((g.n[2] - cz + 1) >> 1);
-    return rows <= 0 ? 0 : (int)((rows + RT_GS_ROWS - 1) / RT_GS_ROWS);
+    if (rows <= 0) return 0;
+    const RowShape w = row_shape<float>(g, rows);
+    return (int)(w.rpw ? (rows + w.rpw - 1) / w.rpw : rows);
 }
 
 template <typename T>
@@ -594,35 +926,33 @@ void launch_fine_gs(const Geom& g, Vec3<T> U, Vec3<const T> F, const float* rhop
     const int cy = pair & 1, cz = pair >> 1;
     const long long rows = (long long)((g.n[1] - cy + 1) >> 1) * ((g.n[2] - cz + 1) >> 1);
     if (rows <= 0) return;
-    dim3 grid((unsigned)((rows + RT_GS_ROWS - 1) / RT_GS_ROWS));
+    if (fu_part && (!reverse || !zero_support || zero_start))
+        throw std::logic_error("f.u partials come from a reverse sweep with zero supports");
+    if (zero_start && (reverse || !zero_support))
+        throw std::logic_error("a zero-start sweep is forward with zero supports");
     const KeC<T> K = kec<T>();
-    if (fu_part) {
-        if (!reverse || !zero_support || zero_start)
-            throw std::logic_error("f.u partials come from a reverse sweep with zero supports");
-        switch (pair) {
-#define RT_CASE(p) case p: hipLaunchKernelGGL((k_fine_gs_pair<T, ((p) & 1), ((p) >> 1), true, true, false, true>), grid, dim3(256), 0, s, g, U, F, rhop, vflag, K, (int)rows, fu_part); break;
-            RT_CASE(0) RT_CASE(1) RT_CASE(2) RT_CASE(3)
+    const RowShape w = row_shape<T>(g, rows);
+    const bool row = w.rpw > 0;
+    const dim3 grid(row ? (unsigned)((rows + w.rpw - 1) / w.rpw) : (unsigned)rows), block(row ? w.nt : 256);
+#define RT_LAUNCH(p, ...)                                                                                            \
+    if (row)                                                                                                         \
+        hipLaunchKernelGGL((k_fine_gs_row<T, ((p) & 1), ((p) >> 1), __VA_ARGS__>), grid, block, 0, s, g, U, F, rhop, \
+                           vflag, K, (int)rows, w.rpw, w.npr, fu_part);                                              \
+    else                                                                                                             \
+        hipLaunchKernelGGL((k_fine_gs_pair<T, ((p) & 1), ((p) >> 1), __VA_ARGS__>), grid, block, 0, s, g, U, F, rhop, \
+                           vflag, K, (int)rows, fu_part);                                                            \
+    break;
+    switch (pair * 8 + (fu_part ? 4 : zero_start ? 5 : (reverse ? 2 : 0) + (zero_support ? 1 : 0))) {
+#define RT_CASE(p)                                          \
+    case p * 8 + 0: RT_LAUNCH(p, false, false)              \
+    case p * 8 + 1: RT_LAUNCH(p, false, true)               \
+    case p * 8 + 2: RT_LAUNCH(p, true, false)               \
+    case p * 8 + 3: RT_LAUNCH(p, true, true)                \
+    case p * 8 + 4: RT_LAUNCH(p, true, true, false, true)   \
+    case p * 8 + 5: RT_LAUNCH(p, false, true, true)
+        RT_CASE(0) RT_CASE(1) RT_CASE(2) RT_CASE(3)
 #undef RT_CASE
-        }
-        RT_HIP(hipGetLastError());
-        return;
-    }
-    if (zero_start) {
-        if (reverse || !zero_support) throw std::logic_error("a zero-start sweep is forward with zero supports");
-        switch (pair) {
-#define RT_CASE(p) case p: hipLaunchKernelGGL((k_fine_gs_pair<T, ((p) & 1), ((p) >> 1), false, true, true>), grid, dim3(256), 0, s, g, U, F, rhop, vflag, K, (int)rows); break;
-            RT_CASE(0) RT_CASE(1) RT_CASE(2) RT_CASE(3)
-#undef RT_CASE
-        }
-        RT_HIP(hipGetLastError());
-        return;
-    }
-    switch (pair * 4 + (reverse ? 2 : 0) + (zero_support ? 1 : 0)) {
-#define RT_CASE(p, r, z) case p * 4 + r * 2 + z: hipLaunchKernelGGL((k_fine_gs_pair<T, ((p) & 1), ((p) >> 1), (r) != 0, (z) != 0>), grid, dim3(256), 0, s, g, U, F, rhop, vflag, K, (int)rows); break;
-        RT_CASE(0, 0, 0) RT_CASE(0, 1, 0) RT_CASE(1, 0, 0) RT_CASE(1, 1, 0) RT_CASE(2, 0, 0) RT_CASE(2, 1, 0)
-        RT_CASE(3, 0, 0) RT_CASE(3, 1, 0) RT_CASE(0, 0, 1) RT_CASE(0, 1, 1) RT_CASE(1, 0, 1) RT_CASE(1, 1, 1)
-        RT_CASE(2, 0, 1) RT_CASE(2, 1, 1) RT_CASE(3, 0, 1) RT_CASE(3, 1, 1)
-#undef RT_CASE
+#undef RT_LAUNCH
     }
     RT_HIP(hipGetLastError());
 }

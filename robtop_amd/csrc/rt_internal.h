@@ -120,7 +120,7 @@ template <typename T>
 void launch_fine_gs(const Geom& g, Vec3<T> U, Vec3<const T> F, const float* rhop, const uint8_t* vflag, int pair,
                     bool reverse, bool zero_support, hipStream_t s, bool zero_start = false,
                     double* fu_part = nullptr);
-int fine_gs_pair_blocks(const Geom& g, int pair);
+int fine_gs_pair_blocks(const Geom& g, int pair);   // FP32
 // one full fine sweep in two launches, old values from Uin, new ones to Uout
 // (Uin is not written; the two must not overlap)
 template <typename T>

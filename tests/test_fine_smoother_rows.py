@@ -1,0 +1,84 @@
+"""The finest smoother's row kernel (one thread per even / odd pair of a row)
+against the tiled smoother, which computes each node by itself: the same bits,
+at the row lengths where the row kernel's workgroups differ: rows of one node
+more than whole waves with and without enough rows to give the node left over
+to the last pair's thread, several rows to a workgroup, rows of part of a wave;
+with holes and with supports inside the solid, so that neighbour checks run."""
+import numpy as np
+import pytest
+
+from robtop_amd.workloads import cube_bits, cube_side
+
+SHAPES = [
+    (128, 96, 96),      # 65 pairs, 2,401 rows a launch: the 65th node goes with the last pair
+    (128, 32, 32),      # 65 pairs, few rows: two waves a row
+    (80, 112, 112),     # 41 pairs, three rows a workgroup
+    (56, 24, 40),       # 29 pairs, one wave a row
+]
+
+
+def problem(ex, ey, ez, seed):
+    import robtop_amd as rt
+    R = cube_side(ex, ey, ez)
+    a = np.zeros((R, R, R), bool)
+    a[:ex, :ey, :ez] = True
+    a[ex // 3:ex // 3 + 3, ey // 2:, :ez // 2] = False
+    a[ex - 1, :, ez // 4] = False
+    hg = rt.HierarchyGrid.genFromMesh(cube_bits(a), R)
+    hg.set_material(1e6, 0.4, 3.0)
+    nx, ny, nz = hg[0].nodes
+    _, vact = hg[0].masks()
+    rng = np.random.default_rng(seed)
+    fixed = np.zeros((nz, ny, nx), bool)
+    fixed[:, :, 0] = True
+    fixed[nz // 2, ny // 2, 5:9] = True
+    fixed[1, 1, nx - 2:] = True
+    fixed = fixed.reshape(-1) & vact
+    hg.set_support(fixed)
+    eact, _ = hg[0].masks()
+    hg.set_density((rng.uniform(0.1, 1.0, eact.size) * eact).astype(np.float32))
+    f = rng.standard_normal((3, vact.size)) * (vact & ~fixed)
+    u = rng.standard_normal((3, vact.size)) * vact
+    return hg, f, u
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("bits", [32, 64])
+def test_sweeps_equal_the_tiled_smoother(shape, bits):
+    print(f"[rows] sweeps {shape} {bits}", flush=True)
+    hg, f, u = problem(*shape, 1)
+    hg.set_precision(bits)
+    out = {}
+    for kind in (0, 1):
+        hg.set_fine_smoother(kind)
+        g = hg[0]
+        g.setForce(f)
+        g.setDisplacement(u)
+        g.gs_relax(1)
+        fwd = g.getDisplacement()
+        g.gs_relax(2, reverse=True)
+        out[kind] = (fwd, g.getDisplacement())
+    assert np.array_equal(out[0][0], out[1][0])
+    assert np.array_equal(out[0][1], out[1][1])
+    assert not np.array_equal(out[0][0], u)
+    hg.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", SHAPES)
+def test_preconditioner_sweeps_equal_the_tiled_smoother(shape):
+    """Zero supports, zero start and reverse sweeps: the FP64 PCG's iterates."""
+    import robtop_amd as rt
+    print(f"[rows] cycles {shape}", flush=True)
+    hg, f, _ = problem(*shape, 2)
+    hg.set_force(f)
+    hg.update_stencil()
+    out = []
+    for kind in (0, 1):
+        hg.set_fine_smoother(kind)
+        hg.set_displacement(np.zeros_like(f))
+        hg.solve(tol=0.0, maxit=3, mode=rt.RT_SOLVE_FP64, pre=2, post=2)
+        out.append(hg.get_displacement())
+    assert np.array_equal(out[0], out[1])
+    hg.close()
