@@ -14,19 +14,49 @@
 // assembled element by element: only elements with some but not all nodes on
 // the island contribute (rigid motions are in the null space of KE).
 //
-// Labels: union-find over the face links of stiff elements (each element
-// unites with its -x, -y and -z neighbours, linking the larger root under the
-// smaller with atomicMin until the link holds), then every element takes its
-// root. Each component ends labelled with its smallest slot, in three passes
-// and no host round trips.
+// Labels: every run of stiff elements along x, cut into segments of 64, takes
+// its smallest slot as label straight from a wave's ballot; then union-find
+// over the remaining face links (linking the larger root under the smaller with
+// atomicMin until the link holds), of two neighbouring rows only where an
+// overlap of their runs begins; then every element takes its root. Each
+// component ends labelled with its smallest slot, without host round trips.
+// One link per overlap in place of one per element is what this costs: at 511 x
+// 256 x 256 elements, most of them one component, the links took 10.7 ms when
+// every element linked its three neighbours.
 #include "rt_internal.h"
 
 namespace rt {
 
-__global__ void k_isl_init(int N, const float* __restrict__ rho, const uint8_t* __restrict__ eflag, float theta,
-                           int* __restrict__ lab) {
-    for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < N; e += gridDim.x * blockDim.x)
-        lab[e] = ((eflag[e] & EF_ACTIVE) && rho[e] >= theta) ? e : -1;
+// one wave per 64-element segment of a row: element (x, y, z) of lane `lane`
+struct Seg { int x, y, z, lane; };
+__device__ __forceinline__ bool seg_at(const Geom& g, long long w, Seg& s) {
+    const int ex = g.n[0] - 1, ey = g.n[1] - 1, ez = g.n[2] - 1, ns = (ex + 63) / 64;
+    if (w >= (long long)ns * ey * ez) return false;
+    const int r = (int)(w / ns);
+    s.lane = (int)__lane_id();
+    s.x = (int)(w % ns) * 64 + s.lane;
+    s.y = r % ey;
+    s.z = r / ey;
+    return true;
+}
+
+// labels of the runs within the segments: the run's smallest slot (its first
+// even element, a run's even elements having the smaller slots), -1 elsewhere.
+// lab holds -1 in every slot on entry.
+__global__ void __launch_bounds__(256) k_isl_rows(Geom g, const float* __restrict__ rho,
+                                                  const uint8_t* __restrict__ eflag, float theta,
+                                                  int* __restrict__ lab) {
+    Seg s;
+    for (long long w = blockIdx.x * 4 + (threadIdx.x >> 6); seg_at(g, w, s); w += gridDim.x * 4) {
+        const bool in = s.x < g.n[0] - 1;
+        const int e = in ? oct_p(g, s.x, s.y, s.z) : 0;
+        const bool stiff = in && (eflag[e] & EF_ACTIVE) && rho[e] >= theta;
+        const unsigned long long m = __ballot(stiff);
+        const unsigned long long gap = ~m & ((1ull << s.lane) - 1);
+        int first = gap ? 64 - __clzll(gap) : 0;
+        if ((first & 1) && first < 63 && (m >> (first + 1) & 1)) first++;
+        if (stiff) lab[e] = oct_p(g, s.x - s.lane + first, s.y, s.z);
+    }
 }
 
 // labels are read with device-scope atomic loads: other workgroups relink
@@ -65,16 +95,20 @@ __device__ __forceinline__ void uf_unite(int* lab, int a, int b) {
     }
 }
 
-__global__ void k_isl_union(Geom g, int* __restrict__ lab) {
-    const int ex = g.n[0] - 1, ey = g.n[1] - 1, ez = g.n[2] - 1;
-    const int tot = ex * ey * ez;
-    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < tot; t += gridDim.x * blockDim.x) {
-        const int x = t % ex, y = (t / ex) % ey, z = t / (ex * ey);
-        const int e = oct_p(g, x, y, z);
-        if (lab[e] < 0) continue;
-        if (x > 0) { const int n = oct_p(g, x - 1, y, z); if (lab[n] >= 0) uf_unite(lab, e, n); }
-        if (y > 0) { const int n = oct_p(g, x, y - 1, z); if (lab[n] >= 0) uf_unite(lab, e, n); }
-        if (z > 0) { const int n = oct_p(g, x, y, z - 1); if (lab[n] >= 0) uf_unite(lab, e, n); }
+__global__ void __launch_bounds__(256) k_isl_union(Geom g, int* __restrict__ lab) {
+    Seg s;
+    for (long long w = blockIdx.x * 4 + (threadIdx.x >> 6); seg_at(g, w, s); w += gridDim.x * 4) {
+        const bool in = s.x < g.n[0] - 1;
+        const int e = in ? oct_p(g, s.x, s.y, s.z) : 0;
+        const bool on = in && lab[e] >= 0;
+        const int ny = in && s.y > 0 ? oct_p(g, s.x, s.y - 1, s.z) : e, nz = in && s.z > 0 ? oct_p(g, s.x, s.y, s.z - 1) : e;
+        const unsigned long long by = __ballot(on && s.y > 0 && lab[ny] >= 0), bz = __ballot(on && s.z > 0 && lab[nz] >= 0);
+        if ((by & ~(by << 1)) >> s.lane & 1) uf_unite(lab, e, ny);
+        if ((bz & ~(bz << 1)) >> s.lane & 1) uf_unite(lab, e, nz);
+        if (on && s.lane == 0 && s.x > 0) {
+            const int n = oct_p(g, s.x - 1, s.y, s.z);
+            if (lab[n] >= 0) uf_unite(lab, e, n);
+        }
     }
 }
 
@@ -84,10 +118,11 @@ __global__ void k_isl_flatten(int N, int* __restrict__ lab) {
 }
 
 // elements with a support node anchor their component. Element counts and
-// anchor flags are aggregated per wave before the atomics: most lanes of a
-// wave share one label (a large component), and one counter hit by every
-// element of the box would serialise.
-__global__ void k_isl_anchor(Geom g, const int* __restrict__ lab, const uint8_t* __restrict__ vflag,
+// anchor flags are aggregated per wave before the atomics (most lanes of a wave
+// share one label), and a component that already counts min_size elements is
+// not counted on: one counter hit by every wave of the box took 5.9 ms at 511 x
+// 256 x 256 elements. count is exact below min_size and at least that otherwise.
+__global__ void k_isl_anchor(Geom g, const int* __restrict__ lab, const uint8_t* __restrict__ vflag, int min_size,
                              uint8_t* __restrict__ anchored, int* __restrict__ count) {
     const int ex = g.n[0] - 1, ey = g.n[1] - 1, ez = g.n[2] - 1;
     const int tot = ex * ey * ez;
@@ -113,8 +148,8 @@ __global__ void k_isl_anchor(Geom g, const int* __restrict__ lab, const uint8_t*
             const unsigned long long m = __ballot(mine);
             const unsigned long long mf = __ballot(mine && fixed);
             if (lane == lead) {
-                atomicAdd(&count[l0], (int)__popcll(m));
-                if (mf) anchored[l0] = 1;
+                if (uf_load(count, l0) < min_size) atomicAdd(&count[l0], (int)__popcll(m));
+                if (mf && !anchored[l0]) anchored[l0] = 1;
             }
             todo = todo && !mine;
         }
@@ -136,10 +171,12 @@ __global__ void k_isl_select(int N, const int* __restrict__ lab, const uint8_t* 
 }
 
 // node -> island: the island of the smallest-numbered island element around the
-// node; support nodes and nodes between two islands get none
+// node; support nodes and nodes between two islands get none. The nodes of all
+// islands are also listed (any order), so that the correction in every cycle
+// visits them alone.
 __global__ void k_isl_nodes(Geom g, const int* __restrict__ lab, const int* __restrict__ root_isl,
                             const uint8_t* __restrict__ vflag, int* __restrict__ node_isl,
-                            double* __restrict__ cent) {
+                            double* __restrict__ cent, int* __restrict__ list, int* __restrict__ nlist) {
     const int nx = g.n[0], ny = g.n[1], nz = g.n[2];
     const int tot = nx * ny * nz;
     for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < tot; t += gridDim.x * blockDim.x) {
@@ -161,6 +198,7 @@ __global__ void k_isl_nodes(Geom g, const int* __restrict__ lab, const int* __re
         if (clash || (vflag[v] & NF_FIXED)) isl = -1;
         node_isl[v] = isl;
         if (isl >= 0) {
+            list[atomicAdd(nlist, 1)] = v;
             atomicAdd(&cent[4 * isl + 0], (double)x);
             atomicAdd(&cent[4 * isl + 1], (double)y);
             atomicAdd(&cent[4 * isl + 2], (double)z);
@@ -299,26 +337,31 @@ __global__ void k_isl_pinv(int nisl, const double* __restrict__ E, double* __res
         }
 }
 
-// zr_i += Z_i^T r over the island's nodes
+// node coordinates of a slot
+__device__ __forceinline__ void slot_xyz(const Geom& g, int v, int& x, int& y, int& z) {
+    const int c = v / g.cs, r = v - c * g.cs;
+    x = 2 * (r % g.h[0]) + (c & 1) - 2;
+    y = 2 * (r / g.h[0] % g.h[1]) + ((c >> 1) & 1) - 2;
+    z = 2 * (r / (g.h[0] * g.h[1])) + (c >> 2) - 2;
+}
+
+// zr_i += Z_i^T r over the islands' nodes
 template <typename T>
-__global__ void k_isl_project(Geom g, const int* __restrict__ node_isl, const double* __restrict__ cent,
-                              Vec3<const T> R, double* __restrict__ zr) {
-    const int nx = g.n[0], ny = g.n[1], nz = g.n[2];
-    const int tot = nx * ny * nz;
-    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < tot; t += gridDim.x * blockDim.x) {
-        const int x = t % nx, y = (t / nx) % ny, z = t / (nx * ny);
-        const int v = oct_p(g, x, y, z);
-        const int i = node_isl[v];
-        if (i < 0) continue;
-        const double r0 = (double)R.c[0][v], r1 = (double)R.c[1][v], r2 = (double)R.c[2][v];
-        const double dx = x - cent[4 * i + 0], dy = y - cent[4 * i + 1], dz = z - cent[4 * i + 2];
-        atomicAdd(&zr[6 * i + 0], r0);
-        atomicAdd(&zr[6 * i + 1], r1);
-        atomicAdd(&zr[6 * i + 2], r2);
-        atomicAdd(&zr[6 * i + 3], dy * r2 - dz * r1);   // (e_x x d) . r
-        atomicAdd(&zr[6 * i + 4], dz * r0 - dx * r2);
-        atomicAdd(&zr[6 * i + 5], dx * r1 - dy * r0);
-    }
+__global__ void k_isl_project(Geom g, int nlist, const int* __restrict__ list, const int* __restrict__ node_isl,
+                              const double* __restrict__ cent, Vec3<const T> R, double* __restrict__ zr) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= nlist) return;
+    const int v = list[t], i = node_isl[v];
+    int x, y, z;
+    slot_xyz(g, v, x, y, z);
+    const double r0 = (double)R.c[0][v], r1 = (double)R.c[1][v], r2 = (double)R.c[2][v];
+    const double dx = x - cent[4 * i + 0], dy = y - cent[4 * i + 1], dz = z - cent[4 * i + 2];
+    atomicAdd(&zr[6 * i + 0], r0);
+    atomicAdd(&zr[6 * i + 1], r1);
+    atomicAdd(&zr[6 * i + 2], r2);
+    atomicAdd(&zr[6 * i + 3], dy * r2 - dz * r1);   // (e_x x d) . r
+    atomicAdd(&zr[6 * i + 4], dz * r0 - dx * r2);
+    atomicAdd(&zr[6 * i + 5], dx * r1 - dy * r0);
 }
 
 // c_i = E_i^+ zr_i, then zr_i = 0 for the next application
@@ -335,44 +378,45 @@ __global__ void k_isl_solve(int nisl, const double* __restrict__ Einv, double* _
     }
 }
 
-// z += Z_i c_i on the island's nodes
+// z += Z_i c_i on the islands' nodes
 template <typename T>
-__global__ void k_isl_correct(Geom g, const int* __restrict__ node_isl, const double* __restrict__ cent,
-                              const double* __restrict__ coef, Vec3<T> Zv) {
-    const int nx = g.n[0], ny = g.n[1], nz = g.n[2];
-    const int tot = nx * ny * nz;
-    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < tot; t += gridDim.x * blockDim.x) {
-        const int x = t % nx, y = (t / nx) % ny, z = t / (nx * ny);
-        const int v = oct_p(g, x, y, z);
-        const int i = node_isl[v];
-        if (i < 0) continue;
-        const double dx = x - cent[4 * i + 0], dy = y - cent[4 * i + 1], dz = z - cent[4 * i + 2];
-        const double* c = coef + 6 * i;
-        // translation + rotation (omega x d), omega = (c3, c4, c5)
-        Zv.c[0][v] += (T)(c[0] + c[4] * dz - c[5] * dy);
-        Zv.c[1][v] += (T)(c[1] + c[5] * dx - c[3] * dz);
-        Zv.c[2][v] += (T)(c[2] + c[3] * dy - c[4] * dx);
-    }
+__global__ void k_isl_correct(Geom g, int nlist, const int* __restrict__ list, const int* __restrict__ node_isl,
+                              const double* __restrict__ cent, const double* __restrict__ coef, Vec3<T> Zv) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= nlist) return;
+    const int v = list[t], i = node_isl[v];
+    int x, y, z;
+    slot_xyz(g, v, x, y, z);
+    const double dx = x - cent[4 * i + 0], dy = y - cent[4 * i + 1], dz = z - cent[4 * i + 2];
+    const double* c = coef + 6 * i;
+    // translation + rotation (omega x d), omega = (c3, c4, c5)
+    Zv.c[0][v] += (T)(c[0] + c[4] * dz - c[5] * dy);
+    Zv.c[1][v] += (T)(c[1] + c[5] * dx - c[3] * dz);
+    Zv.c[2][v] += (T)(c[2] + c[3] * dy - c[4] * dx);
 }
 
 static unsigned grid_for(long long n) { return (unsigned)std::min<long long>((n + 255) / 256, 16384); }
 
 int island_build(const Geom& g, const float* rho, const float* rhop, const uint8_t* eflag, const uint8_t* vflag,
                  const double* KE_dev, float theta, int min_size, int max_isl, int* lab, uint8_t* anchored, int* count,
-                 int* root_isl, int* node_isl, double* cent, double* E, double* Einv, int* flag, hipStream_t s) {
+                 int* root_isl, int* node_isl, double* cent, double* E, double* Einv, int* flag, int* list, int* nlist,
+                 hipStream_t s) {
     const long long ne = (long long)(g.n[0] - 1) * (g.n[1] - 1) * (g.n[2] - 1);
     const long long nn = (long long)g.n[0] * g.n[1] * g.n[2];
-    hipLaunchKernelGGL(k_isl_init, dim3(grid_for(g.N)), dim3(256), 0, s, g.N, rho, eflag, theta, lab);
+    const long long segs = (long long)((g.n[0] + 62) / 64) * (g.n[1] - 1) * (g.n[2] - 1);
+    RT_HIP(hipMemsetAsync(lab, 0xff, sizeof(int) * (size_t)g.N, s));
+    hipLaunchKernelGGL(k_isl_rows, dim3(grid_for(64 * segs)), dim3(256), 0, s, g, rho, eflag, theta, lab);
     RT_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_isl_union, dim3(grid_for(ne)), dim3(256), 0, s, g, lab);
+    hipLaunchKernelGGL(k_isl_union, dim3(grid_for(64 * segs)), dim3(256), 0, s, g, lab);
     RT_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_isl_flatten, dim3(grid_for(g.N)), dim3(256), 0, s, g.N, lab);
     RT_HIP(hipGetLastError());
     RT_HIP(hipMemsetAsync(anchored, 0, (size_t)g.N, s));
     RT_HIP(hipMemsetAsync(count, 0, sizeof(int) * (size_t)g.N, s));
-    hipLaunchKernelGGL(k_isl_anchor, dim3(grid_for(ne)), dim3(256), 0, s, g, lab, vflag, anchored, count);
+    hipLaunchKernelGGL(k_isl_anchor, dim3(grid_for(ne)), dim3(256), 0, s, g, lab, vflag, min_size, anchored,
+                       count);
     RT_HIP(hipGetLastError());
-    RT_HIP(hipMemsetAsync(flag, 0, sizeof(int), s));
+    RT_HIP(hipMemsetAsync(flag, 0, 2 * sizeof(int), s));
     hipLaunchKernelGGL(k_isl_select, dim3(grid_for(g.N)), dim3(256), 0, s, g.N, lab, anchored, count, min_size,
                        max_isl, root_isl, flag);
     RT_HIP(hipGetLastError());
@@ -381,9 +425,12 @@ int island_build(const Geom& g, const float* rho, const float* rhop, const uint8
     RT_HIP(hipStreamSynchronize(s));
     nisl = std::min(nisl, max_isl);
     RT_HIP(hipMemsetAsync(cent, 0, sizeof(double) * 4 * (size_t)std::max(nisl, 1), s));
-    hipLaunchKernelGGL(k_isl_nodes, dim3(grid_for(nn)), dim3(256), 0, s, g, lab, root_isl, vflag, node_isl, cent);
+    hipLaunchKernelGGL(k_isl_nodes, dim3(grid_for(nn)), dim3(256), 0, s, g, lab, root_isl, vflag, node_isl, cent,
+                       list, flag + 1);
     RT_HIP(hipGetLastError());
+    *nlist = 0;
     if (nisl == 0) return 0;
+    RT_HIP(hipMemcpyAsync(nlist, flag + 1, sizeof(int), hipMemcpyDeviceToHost, s));
     hipLaunchKernelGGL(k_isl_centroid, dim3((nisl + 255) / 256), dim3(256), 0, s, nisl, cent);
     RT_HIP(hipMemsetAsync(E, 0, sizeof(double) * 36 * (size_t)nisl, s));
     hipLaunchKernelGGL(k_isl_energy, dim3(grid_for(ne)), dim3(256), 0, s, g, node_isl, rhop, KE_dev, cent, E);
@@ -395,19 +442,19 @@ int island_build(const Geom& g, const float* rho, const float* rhop, const uint8
 }
 
 template <typename T>
-void island_correct(const Geom& g, int nisl, const int* node_isl, const double* cent, const double* Einv, double* zr,
-                    double* coef, Vec3<const T> R, Vec3<T> Zv, hipStream_t s) {
-    if (nisl <= 0) return;
-    const long long nn = (long long)g.n[0] * g.n[1] * g.n[2];
-    hipLaunchKernelGGL((k_isl_project<T>), dim3(grid_for(nn)), dim3(256), 0, s, g, node_isl, cent, R, zr);
+void island_correct(const Geom& g, int nisl, int nlist, const int* list, const int* node_isl, const double* cent,
+                    const double* Einv, double* zr, double* coef, Vec3<const T> R, Vec3<T> Zv, hipStream_t s) {
+    if (nisl <= 0 || nlist <= 0) return;
+    const dim3 grid((unsigned)((nlist + 255) / 256));
+    hipLaunchKernelGGL((k_isl_project<T>), grid, dim3(256), 0, s, g, nlist, list, node_isl, cent, R, zr);
     hipLaunchKernelGGL(k_isl_solve, dim3((nisl + 255) / 256), dim3(256), 0, s, nisl, Einv, zr, coef);
-    hipLaunchKernelGGL((k_isl_correct<T>), dim3(grid_for(nn)), dim3(256), 0, s, g, node_isl, cent, coef, Zv);
+    hipLaunchKernelGGL((k_isl_correct<T>), grid, dim3(256), 0, s, g, nlist, list, node_isl, cent, coef, Zv);
     RT_HIP(hipGetLastError());
 }
 
-template void island_correct<float>(const Geom&, int, const int*, const double*, const double*, double*, double*,
-                                    Vec3<const float>, Vec3<float>, hipStream_t);
-template void island_correct<double>(const Geom&, int, const int*, const double*, const double*, double*, double*,
-                                     Vec3<const double>, Vec3<double>, hipStream_t);
+template void island_correct<float>(const Geom&, int, int, const int*, const int*, const double*, const double*,
+                                    double*, double*, Vec3<const float>, Vec3<float>, hipStream_t);
+template void island_correct<double>(const Geom&, int, int, const int*, const int*, const double*, const double*,
+                                     double*, double*, Vec3<const double>, Vec3<double>, hipStream_t);
 
 }  // namespace rt

@@ -153,7 +153,7 @@ struct Hier {
     int ws_m = 0;                    // solves start from the best combination of the last ws_m solutions (0: off)
     // floating-cluster deflation of the preconditioner (theta <= 0: off)
     float isl_theta = 0.f;
-    int isl_min = 8, isl_max = 4096, nisl = 0;
+    int isl_min = 8, isl_max = 4096, nisl = 0, isl_nodes = 0;   // isl_nodes: listed in isl_cnt
     DBuf isl_lab, isl_anch, isl_cnt, isl_root, isl_node, isl_cent, isl_E, isl_Einv, isl_zr, isl_coef, isl_flag,
         isl_KE;
     std::vector<V3<double>> ws_hist; // ring of previous solutions
@@ -722,8 +722,8 @@ static void vcycle_core(Hier& H, V3<T>& U0, V3<T>& F0, V3<T>& R0, int pre, int p
         for (int v = 0; v < visits; v++) self(self, i + 1);
         prolong_from<T>(H, i, Uv(i), cvt(Uv(i + 1)), zs);
         if (i == 0 && islands)
-            island_correct<T>(H.lv[0].g, H.nisl, H.isl_node.as<int>(), H.isl_cent.as<double>(),
-                              H.isl_Einv.as<double>(), H.isl_zr.as<double>(), H.isl_coef.as<double>(),
+            island_correct<T>(H.lv[0].g, H.nisl, H.isl_nodes, H.isl_cnt.as<int>(), H.isl_node.as<int>(),
+                              H.isl_cent.as<double>(), H.isl_Einv.as<double>(), H.isl_zr.as<double>(), H.isl_coef.as<double>(),
                               cvt(Rv(0)), Uv(0), H.s);
         gs<T>(H, i, Uv(i), Fv(i), post * m, symmetric, zs, false, i == 0 ? fu_part : nullptr);
     };
@@ -1015,14 +1015,14 @@ static void build_islands(Hier& H) {
     H.isl_Einv.ensure(sizeof(double) * 36 * mx);
     if (!H.isl_zr.p) H.isl_zr.alloc(sizeof(double) * 6 * mx);     // zeroed once; the correction leaves it zero
     H.isl_coef.ensure(sizeof(double) * 6 * mx);
-    H.isl_flag.ensure(sizeof(int));
+    H.isl_flag.ensure(2 * sizeof(int));
     H.isl_KE.ensure(sizeof(double) * 576);
     RT_HIP(hipMemcpyAsync(H.isl_KE.p, H.KE, sizeof(double) * 576, hipMemcpyHostToDevice, H.s));
     H.nisl = island_build(L0.g, H.rho.as<float>(), H.rhop.as<float>(), H.eflag.as<uint8_t>(), L0.vflag.as<uint8_t>(),
                           H.isl_KE.as<double>(), H.isl_theta, H.isl_min, H.isl_max, H.isl_lab.as<int>(),
                           H.isl_anch.as<uint8_t>(), H.isl_cnt.as<int>(), H.isl_root.as<int>(), H.isl_node.as<int>(),
                           H.isl_cent.as<double>(), H.isl_E.as<double>(), H.isl_Einv.as<double>(),
-                          H.isl_flag.as<int>(), H.s);
+                          H.isl_flag.as<int>(), H.isl_cnt.as<int>(), &H.isl_nodes, H.s);   // (the counts are used up)
 }
 
 static void update_stencil(Hier& H) {
@@ -2774,8 +2774,8 @@ static void vcycle_batch(Hier& H, int nb, int pre, int post) {
         for (int b = 0; b < nb; b++) prolong_from<float>(H, i, L.bU.v(b), C.bU.cv(b), i == 0);
         if (i == 0)
             for (int b = 0; b < nb; b++)
-                island_correct<float>(L.g, H.nisl, H.isl_node.as<int>(), H.isl_cent.as<double>(),
-                                      H.isl_Einv.as<double>(), H.isl_zr.as<double>(), H.isl_coef.as<double>(),
+                island_correct<float>(L.g, H.nisl, H.isl_nodes, H.isl_cnt.as<int>(), H.isl_node.as<int>(),
+                                      H.isl_cent.as<double>(), H.isl_Einv.as<double>(), H.isl_zr.as<double>(), H.isl_coef.as<double>(),
                                       L.bR.cv(b), L.bU.v(b), H.s);
         smooth(i, post * m, true, false);
     };

@@ -194,14 +194,16 @@ void launch_lincomb(double* x, const double* const* h, const double* c, int k, s
 // floating-cluster deflation (k_island.hip): builds the islands of stiff
 // elements (rho >= theta, at least min_size elements, at most max_isl) that
 // touch no support, their centroids and pseudo-inverted rigid-body energies;
-// returns the island count
+// returns the island count; list (N slots) gets the islands' nodes, *nlist of
+// them. flag: two ints of device scratch.
 int island_build(const Geom& g, const float* rho, const float* rhop, const uint8_t* eflag, const uint8_t* vflag,
                  const double* KE_dev, float theta, int min_size, int max_isl, int* lab, uint8_t* anchored, int* count,
-                 int* root_isl, int* node_isl, double* cent, double* E, double* Einv, int* flag, hipStream_t s);
+                 int* root_isl, int* node_isl, double* cent, double* E, double* Einv, int* flag, int* list, int* nlist,
+                 hipStream_t s);
 // Z += sum_i Z_i E_i^+ Z_i^T R (zr must be zero on entry and is left zero)
 template <typename T>
-void island_correct(const Geom& g, int nisl, const int* node_isl, const double* cent, const double* Einv, double* zr,
-                    double* coef, Vec3<const T> R, Vec3<T> Zv, hipStream_t s);
+void island_correct(const Geom& g, int nisl, int nlist, const int* list, const int* node_isl, const double* cent,
+                    const double* Einv, double* zr, double* coef, Vec3<const T> R, Vec3<T> Zv, hipStream_t s);
 // b = a rounded to bfloat16 (round to nearest even, through binary32)
 void launch_to_bf16(const double* a, bf16* b, size_t n, hipStream_t s);
 template <typename TA, typename TB>
