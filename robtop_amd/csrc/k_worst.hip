@@ -106,4 +106,92 @@ void launch_pm_commit(int nl, const int* slots, const double* fs, double scale, 
     RT_HIP(hipGetLastError());
 }
 
+// ---------------------------------------------------------------------------
+// C = A^T B for tall A (m x na) and B (m x nb), column-major, both of a few
+// columns: the block Lanczos projections. A GEMM of this shape has one output
+// tile and runs its whole length of m in one workgroup (9.4 ms at m = 150,000,
+// 8 x 8); here the rows are cut into chunks, each workgroup takes 4 x 4 columns
+// of one chunk, and the chunks' partial sums are added in order.
+// Bound: the reads, a column of A once per four columns of B and the other way
+// round, from HBM the first time and from L2 after that.
+// ---------------------------------------------------------------------------
+namespace {
+constexpr int kGramRows = 2048;     // rows of a chunk: eight per thread
+constexpr int kGramTile = 4;
+}  // namespace
+
+__global__ void __launch_bounds__(256) k_gram(int m, int na, int nb, const double* __restrict__ A,
+                                              const double* __restrict__ B, double* __restrict__ part) {
+    __shared__ double red[4][kGramTile * kGramTile];
+    const int ta = (na + kGramTile - 1) / kGramTile;
+    const int i0 = (blockIdx.y % ta) * kGramTile, j0 = (blockIdx.y / ta) * kGramTile;
+    // columns past the last one repeat it; their sums are dropped
+    const double *a[kGramTile], *b[kGramTile];
+#pragma unroll
+    for (int k = 0; k < kGramTile; k++) {
+        a[k] = A + (size_t)min(i0 + k, na - 1) * m;
+        b[k] = B + (size_t)min(j0 + k, nb - 1) * m;
+    }
+    double acc[kGramTile][kGramTile] = {};
+    const int r1 = min((int)(blockIdx.x + 1) * kGramRows, m);
+    for (int r = blockIdx.x * kGramRows + threadIdx.x; r < r1; r += 256) {
+        double x[kGramTile], y[kGramTile];
+#pragma unroll
+        for (int k = 0; k < kGramTile; k++) { x[k] = a[k][r]; y[k] = b[k][r]; }
+#pragma unroll
+        for (int i = 0; i < kGramTile; i++)
+#pragma unroll
+            for (int j = 0; j < kGramTile; j++) acc[i][j] += x[i] * y[j];
+    }
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+    for (int i = 0; i < kGramTile; i++)
+#pragma unroll
+        for (int j = 0; j < kGramTile; j++) {
+            double v = acc[i][j];
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+            if (lane == 0) red[w][kGramTile * j + i] = v;
+        }
+    __syncthreads();
+    const int t = threadIdx.x;
+    if (t < kGramTile * kGramTile)
+        part[((size_t)blockIdx.y * gridDim.x + blockIdx.x) * kGramTile * kGramTile + t] =
+            (red[0][t] + red[1][t]) + (red[2][t] + red[3][t]);
+}
+
+// one workgroup per tile: entry t % 16, chunks t / 16, t / 16 + 16, ...
+__global__ void __launch_bounds__(256) k_gram_sum(int chunks, int na, int nb, const double* __restrict__ part,
+                                                  double* __restrict__ C) {
+    __shared__ double red[16][16];
+    const int e = threadIdx.x & 15, q = threadIdx.x >> 4;
+    const double* p = part + (size_t)blockIdx.x * chunks * 16;
+    double v = 0;
+    for (int c = q; c < chunks; c += 16) v += p[(size_t)c * 16 + e];
+    red[q][e] = v;
+    __syncthreads();
+    if (q) return;
+    double t = 0;
+#pragma unroll
+    for (int k = 0; k < 16; k++) t += red[k][e];
+    const int ta = (na + kGramTile - 1) / kGramTile;
+    const int i = (blockIdx.x % ta) * kGramTile + e % kGramTile, j = (blockIdx.x / ta) * kGramTile + e / kGramTile;
+    if (i < na && j < nb) C[(size_t)j * na + i] = t;
+}
+
+static int gram_tiles(int na, int nb) {
+    return ((na + kGramTile - 1) / kGramTile) * ((nb + kGramTile - 1) / kGramTile);
+}
+static int gram_chunks(int m) { return (m + kGramRows - 1) / kGramRows; }
+size_t gram_work(int m, int na, int nb) {
+    return (size_t)gram_tiles(na, nb) * gram_chunks(m) * kGramTile * kGramTile;
+}
+void launch_gram(int m, int na, int nb, const double* A, const double* B, double* C, double* work, hipStream_t s) {
+    if (m < 1 || na < 1 || nb < 1) throw std::invalid_argument("launch_gram: empty operand");
+    const int tiles = gram_tiles(na, nb), chunks = gram_chunks(m);
+    hipLaunchKernelGGL(k_gram, dim3(chunks, tiles), dim3(256), 0, s, m, na, nb, A, B, work);
+    hipLaunchKernelGGL(k_gram_sum, dim3(tiles), dim3(256), 0, s, chunks, na, nb, (const double*)work, C);
+    RT_HIP(hipGetLastError());
+}
+
 }  // namespace rt

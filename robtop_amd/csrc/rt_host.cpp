@@ -126,6 +126,7 @@ struct Hier {
     // worst-case load search: load-node slots, unit normals (constrained
     // direction), projected force and the previous step's force, all [3][nload]
     DBuf load_slots, load_nrm, pm_fs, pm_old;
+    DBuf gram;                       // block Lanczos: partial sums of the projections
     // no-support modes: the admissible rigid motions of the load nodes
     // (compact [k][c * nload + i], nrd of them) and the finest nodes' rigid
     // motions (6 vectors, built on first use)
@@ -2637,6 +2638,12 @@ static void dscal(Hier& H, int n, double a, double* x) {
     if (rocblas_dscal(H.blas, n, &a, x, 1) != rocblas_status_success) throw std::runtime_error("rocblas_dscal failed");
 }
 
+// C = A^T B (launch_gram) with the handle's workspace
+static void gram(Hier& H, int m, int na, int nb, const double* A, const double* B, double* C) {
+    H.gram.ensure(sizeof(double) * gram_work(m, na, nb));
+    launch_gram(m, na, nb, A, B, C, H.gram.as<double>(), H.s);
+}
+
 // Orthonormalises the k columns of W (m x k, device) against the first nq
 // columns of Q (two classical Gram-Schmidt passes as GEMMs), then among
 // themselves (modified Gram-Schmidt, two passes). W_in = Q C + W_out R with R
@@ -2648,7 +2655,7 @@ static int block_orth_dev(Hier& H, int m, int k, double* W, const double* Q, int
     for (int j = 0; j < k; j++) n0[j] = std::sqrt(std::max(0.0, ddot(H, m, W + (size_t)j * m, W + (size_t)j * m)));
     if (nq > 0)
         for (int pass = 0; pass < 2; pass++) {
-            gemm(H, rocblas_operation_transpose, rocblas_operation_none, nq, k, m, 1.0, Q, m, W, m, 0.0, C, nq);
+            gram(H, m, nq, k, Q, W, C);
             gemm(H, rocblas_operation_none, rocblas_operation_none, m, k, nq, -1.0, Q, m, C, nq, 1.0, W, m);
         }
     R.assign((size_t)k * k, 0.0);
@@ -3117,6 +3124,7 @@ static double block_lanczos(Hier& H, int k, int max_blocks, double tol, double s
     Cd.alloc(sizeof(double) * (size_t)(max_blocks + 1) * k * k);
     Md.alloc(sizeof(double) * (size_t)k * k);
     fd.alloc(sizeof(double) * m);
+    H.gram.ensure(sizeof(double) * gram_work(mi, max_blocks * k, k));
     double* Q = Qd.as<double>();
     auto col = [&](int c) { return Q + (size_t)c * m; };
     // seeded start block (splitmix64 uniforms in [-1, 1)), projected per load node onto n n^T
@@ -3168,7 +3176,7 @@ static double block_lanczos(Hier& H, int k, int max_blocks, double tol, double s
         }
         // A_j = Q_j^T W (symmetrised); column-major k x k, A(a, b) = q_a . w_b
         std::vector<double> A((size_t)k * k);
-        gemm(H, rocblas_operation_transpose, rocblas_operation_none, k, k, mi, 1.0, blk, mi, W, mi, 0.0, Md.as<double>(), k);
+        gram(H, mi, k, k, blk, W, Md.as<double>());
         RT_HIP(hipMemcpyAsync(A.data(), Md.p, sizeof(double) * k * k, hipMemcpyDeviceToHost, H.s));
         RT_HIP(hipStreamSynchronize(H.s));
         for (int a = 0; a < k; a++)

@@ -280,6 +280,11 @@ void launch_pm_gather(int nl, const int* slots, Vec3<const double> X, const doub
 void launch_pm_commit(int nl, const int* slots, const double* fs, double scale, Vec3<double> F, double* fold,
                       double* partials, int nparts, hipStream_t s);
 
+// C (na x nb) = A^T B, A m x na, B m x nb, column-major without padding; work:
+// gram_work(m, na, nb) doubles
+size_t gram_work(int m, int na, int nb);
+void launch_gram(int m, int na, int nb, const double* A, const double* B, double* C, double* work, hipStream_t s);
+
 // k_voxel.hip
 void launch_voxelize(const float* tris, int ntris, const float bmin[3], const float unit[3], int R, uint32_t* bits,
                      hipStream_t s);
