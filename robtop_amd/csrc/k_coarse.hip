@@ -471,6 +471,8 @@ template <typename T, int RATIO>
 __global__ void __launch_bounds__(256) k_restrict(Geom gf, int ofx, int ofy, int ofz, Vec3<const T> Rf, Geom gc,
                                                   int ocx, int ocy, int ocz, Vec3<T> Fc,
                                                   const uint8_t* __restrict__ vflag_c) {
+    at_batch(Rf, blockIdx.y, 3 * gf.N);
+    at_batch(Fc, blockIdx.y, 3 * gc.N);
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     const int ncx = gc.n[0], ncy = gc.n[1], ncz = gc.n[2];
     if (t >= ncx * ncy * ncz) return;
@@ -521,6 +523,8 @@ __global__ void __launch_bounds__(256) k_restrict_xy(Geom gf, int ofx, int ofy, 
                                                      int ocx, int ocy, T* __restrict__ W) {
     __shared__ T row[3][kProlongRowMax];
     const int nx = gf.n[0], ny = gf.n[1], nz = gf.n[2];
+    at_batch(Rf, blockIdx.y, 3 * gf.N);
+    W += (size_t)blockIdx.y * 3 * ncx * ncy * nz;
     const int b = xcd_row(blockIdx.x, gridDim.x);
     const int yc = b % ncy, z = b / ncy;
     const int fy = (ocy + yc) * RATIO - ofy;
@@ -600,6 +604,8 @@ __global__ void __launch_bounds__(256) k_restrict_z(int nfz, int ofz, const T* _
                                                     Vec3<T> Fc, const uint8_t* __restrict__ vflag_c) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     const int ncx = gc.n[0], ncy = gc.n[1];
+    at_batch(Fc, blockIdx.y, 3 * gc.N);
+    W += (size_t)blockIdx.y * 3 * ncx * ncy * nfz;
     if (t >= ncx * ncy * gc.n[2]) return;
     const int xy = t % (ncx * ncy), zc = t / (ncx * ncy);
     const int vc = oct_p(gc, xy % ncx, xy / ncx, zc);
@@ -628,12 +634,12 @@ size_t restrict_scratch_elems(const Geom& gf, const Geom& gc) {
 
 template <typename T>
 void launch_restrict(const Geom& gf, const int of[3], Vec3<const T> Rf, const Geom& gc, const int oc[3], Vec3<T> Fc,
-                     const uint8_t* vflag_c, int ratio, T* scratch, hipStream_t s) {
+                     const uint8_t* vflag_c, int ratio, T* scratch, hipStream_t s, int nb) {
     long long tot = (long long)gc.n[0] * gc.n[1] * gc.n[2];
-    dim3 grid((unsigned)((tot + 255) / 256));
+    dim3 grid((unsigned)((tot + 255) / 256), nb);
     if (ratio == 4 && scratch && gf.n[0] <= kProlongRowMax) {
         const long long wgs = (long long)gc.n[1] * gf.n[2];
-        hipLaunchKernelGGL((k_restrict_xy<T, 4>), dim3((unsigned)wgs), dim3(256), 0, s, gf, of[0], of[1], Rf,
+        hipLaunchKernelGGL((k_restrict_xy<T, 4>), dim3((unsigned)wgs, nb), dim3(256), 0, s, gf, of[0], of[1], Rf,
                            gc.n[0], gc.n[1], oc[0], oc[1], scratch);
         RT_HIP(hipGetLastError());
         hipLaunchKernelGGL((k_restrict_z<T, 4>), grid, dim3(256), 0, s, gf.n[2], of[2], (const T*)scratch, gc, oc[2],
@@ -654,6 +660,8 @@ __global__ void __launch_bounds__(256) k_prolong(Geom gf, int ofx, int ofy, int 
                                                  int ocz, Vec3<const T> Uc, int skip_fixed) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     const int nx = gf.n[0], ny = gf.n[1], nz = gf.n[2];
+    at_batch(Uf, blockIdx.y, 3 * gf.N);
+    at_batch(Uc, blockIdx.y, 3 * gc.N);
     if (t >= nx * ny * nz) return;
     const int x = t % nx, y = (t / nx) % ny, z = t / (nx * ny);
     const int v = oct_p(gf, x, y, z);
@@ -694,6 +702,8 @@ __global__ void __launch_bounds__(256) k_prolong_row(Geom gf, int ofx, int ofy, 
     constexpr int H = kProlongRowMax / 2;
     __shared__ T inc[3][2][H];
     const int nx = gf.n[0], ny = gf.n[1];
+    at_batch(Uf, blockIdx.y, 3 * gf.N);
+    at_batch(Uc, blockIdx.y, 3 * gc.N);
     const int y = blockIdx.x % ny, z = blockIdx.x / ny;
     const int ay = ofy + y, az = ofz + z;
     const int py = ay % RATIO, pz = az % RATIO;
@@ -770,19 +780,19 @@ __global__ void __launch_bounds__(256) k_prolong_row(Geom gf, int ofx, int ofy, 
 
 template <typename T>
 void launch_prolong(const Geom& gf, const int of[3], Vec3<T> Uf, const uint8_t* vflag_f, const Geom& gc,
-                    const int oc[3], Vec3<const T> Uc, int ratio, bool skip_fixed, hipStream_t s) {
+                    const int oc[3], Vec3<const T> Uc, int ratio, bool skip_fixed, hipStream_t s, int nb) {
     if (ratio == 4 && gf.n[0] <= kProlongRowMax) {
         const int gx0 = of[0] / 4, ngx = (of[0] + gf.n[0] - 1) / 4 - gx0 + 1;
         const long long rows = (long long)gf.n[1] * gf.n[2];
-        hipLaunchKernelGGL((k_prolong_row<T, 4>), dim3((unsigned)rows), dim3(256), 0, s, gf, of[0], of[1], of[2], Uf,
+        hipLaunchKernelGGL((k_prolong_row<T, 4>), dim3((unsigned)rows, nb), dim3(256), 0, s, gf, of[0], of[1], of[2], Uf,
                            vflag_f, gc, oc[0], oc[1], oc[2], Uc, (int)skip_fixed, gx0, ngx);
     } else if (ratio == 4) {
         long long tot = (long long)gf.n[0] * gf.n[1] * gf.n[2];
-        hipLaunchKernelGGL((k_prolong<T, 4>), dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, gf, of[0], of[1],
+        hipLaunchKernelGGL((k_prolong<T, 4>), dim3((unsigned)((tot + 255) / 256), nb), dim3(256), 0, s, gf, of[0], of[1],
                            of[2], Uf, vflag_f, gc, oc[0], oc[1], oc[2], Uc, (int)skip_fixed);
     } else {
         long long tot = (long long)gf.n[0] * gf.n[1] * gf.n[2];
-        hipLaunchKernelGGL((k_prolong<T, 2>), dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, gf, of[0], of[1],
+        hipLaunchKernelGGL((k_prolong<T, 2>), dim3((unsigned)((tot + 255) / 256), nb), dim3(256), 0, s, gf, of[0], of[1],
                            of[2], Uf, vflag_f, gc, oc[0], oc[1], oc[2], Uc, (int)skip_fixed);
     }
     RT_HIP(hipGetLastError());
@@ -914,11 +924,14 @@ __device__ __forceinline__ double blk_sum(double v) {
 // chunk (optional): one byte per 1024 float4 (4096 floats) of the vectors,
 // 0 where every value is known to be 0 (no active node): those are skipped,
 // which leaves every sum and vector unchanged
+// (blockIdx.y: vector of a batch, n apart, partials pstride apart; so in the
+// other vector kernels)
 __global__ void __launch_bounds__(256) k_dot4_partials(const float* __restrict__ a, const float* __restrict__ b,
                                                        size_t n4, double* __restrict__ partials,
-                                                       const uint8_t* __restrict__ chunk) {
-    const float4* a4 = reinterpret_cast<const float4*>(a);
-    const float4* b4 = reinterpret_cast<const float4*>(b);
+                                                       const uint8_t* __restrict__ chunk, int pstride) {
+    const float4* a4 = reinterpret_cast<const float4*>(a) + blockIdx.y * n4;
+    const float4* b4 = reinterpret_cast<const float4*>(b) + blockIdx.y * n4;
+    partials += (size_t)blockIdx.y * pstride;
     double s = 0;
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n4; i += (size_t)gridDim.x * blockDim.x) {
         if (chunk && !chunk[i >> 10]) continue;
@@ -931,7 +944,10 @@ __global__ void __launch_bounds__(256) k_dot4_partials(const float* __restrict__
 
 template <typename TA, typename TB>
 __global__ void __launch_bounds__(256) k_dot_partials(const TA* __restrict__ a, const TB* __restrict__ b, size_t n,
-                                                      double* __restrict__ partials) {
+                                                      double* __restrict__ partials, int pstride) {
+    a += blockIdx.y * n;
+    b += blockIdx.y * n;
+    partials += (size_t)blockIdx.y * pstride;
     double s = 0;
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
         s += (double)a[i] * (double)b[i];
@@ -941,19 +957,19 @@ __global__ void __launch_bounds__(256) k_dot_partials(const TA* __restrict__ a, 
 
 template <typename TA, typename TB>
 void launch_dot_partials_t(const TA* a, const TB* b, size_t n, double* partials, int nparts, hipStream_t s,
-                           const uint8_t* chunk) {
+                           const uint8_t* chunk, int nb, int pstride) {
     if constexpr (std::is_same<TA, float>::value && std::is_same<TB, float>::value) {
         if (n % 4 == 0) {
-            hipLaunchKernelGGL(k_dot4_partials, dim3(nparts), dim3(256), 0, s, a, b, n / 4, partials, chunk);
+            hipLaunchKernelGGL(k_dot4_partials, dim3(nparts, nb), dim3(256), 0, s, a, b, n / 4, partials, chunk, pstride);
             RT_HIP(hipGetLastError());
             return;
         }
     }
-    hipLaunchKernelGGL((k_dot_partials<TA, TB>), dim3(nparts), dim3(256), 0, s, a, b, n, partials);
+    hipLaunchKernelGGL((k_dot_partials<TA, TB>), dim3(nparts, nb), dim3(256), 0, s, a, b, n, partials, pstride);
     RT_HIP(hipGetLastError());
 }
 void launch_dot_partials(const double* a, const double* b, size_t n, double* partials, int nparts, hipStream_t s) {
-    launch_dot_partials_t<double, double>(a, b, n, partials, nparts, s, nullptr);
+    launch_dot_partials_t<double, double>(a, b, n, partials, nparts, s);
 }
 
 // chunk mask of a finest-level vector (3 components of N slots): byte c = 1 if
@@ -971,7 +987,9 @@ void launch_vec_chunks(const uint8_t* vflag, int N, uint8_t* chunk, hipStream_t 
 
 // one workgroup of 1024 threads; each thread keeps four running sums over
 // interleaved runs of the partials (independent loads in flight, fixed order)
-__global__ void __launch_bounds__(1024) k_sum_partials(const double* __restrict__ p, int n, double* __restrict__ out) {
+__global__ void __launch_bounds__(1024) k_sum_partials(const double* __restrict__ p, int n, double* __restrict__ out,
+                                                       int pstride) {
+    p += (size_t)blockIdx.x * pstride;
     double a[4] = {0, 0, 0, 0};
     const int step = 4 * (int)blockDim.x;
     for (int i = threadIdx.x; i < n; i += step) {
@@ -983,19 +1001,23 @@ __global__ void __launch_bounds__(1024) k_sum_partials(const double* __restrict_
     }
     double s = (a[0] + a[1]) + (a[2] + a[3]);
     s = blk_sum(s);
-    if (threadIdx.x == 0) out[0] = s;
+    if (threadIdx.x == 0) out[blockIdx.x] = s;
 }
-void launch_sum_partials(const double* partials, int nparts, double* out, hipStream_t s) {
-    hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(1024), 0, s, partials, nparts, out);
+void launch_sum_partials(const double* partials, int nparts, double* out, hipStream_t s, int nb, int pstride) {
+    hipLaunchKernelGGL(k_sum_partials, dim3(nb), dim3(1024), 0, s, partials, nparts, out, pstride);
     RT_HIP(hipGetLastError());
 }
 
 // x += a p; r -= a q; partials of r.r; rz = (TZ) r
 template <typename T, typename TZ>
 __global__ void __launch_bounds__(256) k_pcg_xr(T* __restrict__ x, T* __restrict__ r, const T* __restrict__ p,
-                                                const T* __restrict__ q, double alpha, size_t n,
-                                                double* __restrict__ partials, TZ* __restrict__ rz) {
-    const T a = (T)alpha;
+                                                const T* __restrict__ q, Coefs alpha, size_t n,
+                                                double* __restrict__ partials, TZ* __restrict__ rz, int pstride) {
+    const size_t o = blockIdx.y * n;
+    x += o; r += o; p += o; q += o;
+    if (rz) rz += o;
+    partials += (size_t)blockIdx.y * pstride;
+    const T a = (T)alpha.v[blockIdx.y];
     double s = 0;
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
         x[i] += a * p[i];
@@ -1008,27 +1030,25 @@ __global__ void __launch_bounds__(256) k_pcg_xr(T* __restrict__ x, T* __restrict
     if (threadIdx.x == 0) partials[blockIdx.x] = s;
 }
 template <typename T, typename TZ>
-void launch_pcg_update_x_r(T* x, T* r, const T* p, const T* q, double alpha, size_t n, double* partials, int nparts,
-                           TZ* rz_out, hipStream_t s) {
-    hipLaunchKernelGGL((k_pcg_xr<T, TZ>), dim3(nparts), dim3(256), 0, s, x, r, p, q, alpha, n, partials, rz_out);
+void launch_pcg_update_x_r(T* x, T* r, const T* p, const T* q, Coefs alpha, size_t n, double* partials, int nparts,
+                           TZ* rz_out, hipStream_t s, int nb, int pstride) {
+    hipLaunchKernelGGL((k_pcg_xr<T, TZ>), dim3(nparts, nb), dim3(256), 0, s, x, r, p, q, alpha, n, partials, rz_out,
+                       pstride);
     RT_HIP(hipGetLastError());
 }
 
-// reliable-update PCG step: r (FP32) -= a q with partials of r.r, and, when
-// DX, the FP32 solution increment dx += a p in the same pass.
+// reliable-update PCG step: r (FP32) -= a q with partials of r.r.
 // The FP32 streaming kernels of the reliable-update PCG take four values per
 // lane per step (16 B loads) when n is a multiple of 4 (it is: n = 3 * 8 cs),
 // over kStreamBlocks workgroups, so enough bytes are in flight to approach
 // the HBM rate.
-template <bool DX>
-__global__ void __launch_bounds__(256) k_pcg_ru_dxr(float* __restrict__ r, const float* __restrict__ q,
-                                                    float* __restrict__ dx, const float* __restrict__ p, float a,
-                                                    size_t n4, double* __restrict__ partials,
-                                                    const uint8_t* __restrict__ chunk) {
-    float4* r4 = reinterpret_cast<float4*>(r);
-    float4* d4 = reinterpret_cast<float4*>(dx);
-    const float4* q4 = reinterpret_cast<const float4*>(q);
-    const float4* p4 = reinterpret_cast<const float4*>(p);
+__global__ void __launch_bounds__(256) k_pcg_ru_r(float* __restrict__ r, const float* __restrict__ q, Coefs alpha,
+                                                  size_t n4, double* __restrict__ partials,
+                                                  const uint8_t* __restrict__ chunk, int pstride) {
+    float4* r4 = reinterpret_cast<float4*>(r) + blockIdx.y * n4;
+    const float4* q4 = reinterpret_cast<const float4*>(q) + blockIdx.y * n4;
+    partials += (size_t)blockIdx.y * pstride;
+    const float a = (float)alpha.v[blockIdx.y];
     double s = 0;
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n4; i += (size_t)gridDim.x * blockDim.x) {
         if (chunk && !chunk[i >> 10]) continue;
@@ -1036,28 +1056,15 @@ __global__ void __launch_bounds__(256) k_pcg_ru_dxr(float* __restrict__ r, const
         const float4 qi = q4[i];
         ri.x -= a * qi.x; ri.y -= a * qi.y; ri.z -= a * qi.z; ri.w -= a * qi.w;
         r4[i] = ri;
-        if constexpr (DX) {
-            const float4 pi = p4[i];
-            float4 di = d4[i];
-            di.x += a * pi.x; di.y += a * pi.y; di.z += a * pi.z; di.w += a * pi.w;
-            d4[i] = di;
-        }
         s += ((double)ri.x * ri.x + (double)ri.y * ri.y) + ((double)ri.z * ri.z + (double)ri.w * ri.w);
     }
     s = blk_sum(s);
     if (threadIdx.x == 0) partials[blockIdx.x] = s;
 }
-void launch_pcg_ru_dxr(float* r, const float* q, float* dx, const float* p, double alpha, size_t n, double* partials,
-                       int nparts, hipStream_t s, const uint8_t* chunk) {
-    if (n % 4) throw std::logic_error("launch_pcg_ru_dxr: n must be a multiple of 4");
-    if (dx) {
-        if (!p) throw std::logic_error("launch_pcg_ru_dxr: dx without p");
-        hipLaunchKernelGGL(k_pcg_ru_dxr<true>, dim3(nparts), dim3(256), 0, s, r, q, dx, p, (float)alpha, n / 4,
-                           partials, chunk);
-    } else {
-        hipLaunchKernelGGL(k_pcg_ru_dxr<false>, dim3(nparts), dim3(256), 0, s, r, q, dx, p, (float)alpha, n / 4,
-                           partials, chunk);
-    }
+void launch_pcg_ru_r(float* r, const float* q, Coefs alpha, size_t n, double* partials, int nparts, hipStream_t s,
+                     const uint8_t* chunk, int nb, int pstride) {
+    if (n % 4) throw std::logic_error("launch_pcg_ru_r: n must be a multiple of 4");
+    hipLaunchKernelGGL(k_pcg_ru_r, dim3(nparts, nb), dim3(256), 0, s, r, q, alpha, n / 4, partials, chunk, pstride);
     RT_HIP(hipGetLastError());
 }
 
@@ -1079,66 +1086,50 @@ void launch_pcg_flush_x(double* x, float* dx, size_t n, hipStream_t s, const flo
 }
 
 // dx += a p, then p = z + b p: the direction update with the previous step's
-// solution increment, deferred from k_pcg_ru_dxr so that p is read once for
-// both (same FP32 operations, so the same bits as updating dx with r)
-__global__ void __launch_bounds__(256) k_pcg_p4_dx(float* __restrict__ p, const float* __restrict__ z, float b,
-                                                   float* __restrict__ dx, float a, size_t n4,
+// solution increment, deferred from k_pcg_ru_r so that p is read once for both
+// (same FP32 operations, so the same bits as updating dx with r). a = 0: no
+// increment is pending, dx is left alone.
+__global__ void __launch_bounds__(256) k_pcg_p4_dx(float* __restrict__ p, const float* __restrict__ z, Coefs beta,
+                                                   float* __restrict__ dx, Coefs alpha, size_t n4,
                                                    const uint8_t* __restrict__ chunk) {
-    float4* p4 = reinterpret_cast<float4*>(p);
-    float4* d4 = reinterpret_cast<float4*>(dx);
-    const float4* z4 = reinterpret_cast<const float4*>(z);
+    float4* p4 = reinterpret_cast<float4*>(p) + blockIdx.y * n4;
+    float4* d4 = reinterpret_cast<float4*>(dx) + blockIdx.y * n4;
+    const float4* z4 = reinterpret_cast<const float4*>(z) + blockIdx.y * n4;
+    const float b = (float)beta.v[blockIdx.y], a = (float)alpha.v[blockIdx.y];
+    const bool add = alpha.v[blockIdx.y] != 0.0;
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n4; i += (size_t)gridDim.x * blockDim.x) {
         if (chunk && !chunk[i >> 10]) continue;
         const float4 zi = z4[i];
         float4 pi = p4[i];
-        float4 di = d4[i];
-        di.x += a * pi.x; di.y += a * pi.y; di.z += a * pi.z; di.w += a * pi.w;
+        if (add) {
+            float4 di = d4[i];
+            di.x += a * pi.x; di.y += a * pi.y; di.z += a * pi.z; di.w += a * pi.w;
+            d4[i] = di;
+        }
         pi.x = zi.x + b * pi.x; pi.y = zi.y + b * pi.y; pi.z = zi.z + b * pi.z; pi.w = zi.w + b * pi.w;
-        d4[i] = di;
         p4[i] = pi;
     }
 }
-void launch_pcg_p_dx(float* p, const float* z, double beta, float* dx, double alpha, size_t n, hipStream_t s,
-                     const uint8_t* chunk) {
+void launch_pcg_p_dx(float* p, const float* z, Coefs beta, float* dx, Coefs alpha, size_t n, hipStream_t s,
+                     const uint8_t* chunk, int nb) {
     if (n % 4) throw std::logic_error("launch_pcg_p_dx: n must be a multiple of 4");
-    hipLaunchKernelGGL(k_pcg_p4_dx, dim3(kStreamBlocks), dim3(256), 0, s, p, z, (float)beta, dx, (float)alpha, n / 4,
-                       chunk);
+    hipLaunchKernelGGL(k_pcg_p4_dx, dim3(kStreamBlocks, nb), dim3(256), 0, s, p, z, beta, dx, alpha, n / 4, chunk);
     RT_HIP(hipGetLastError());
 }
 
-// p = z + b p, four FP32 values per lane
-__global__ void __launch_bounds__(256) k_pcg_p4(float* __restrict__ p, const float* __restrict__ z, float b,
-                                                size_t n4, const uint8_t* __restrict__ chunk) {
-    float4* p4 = reinterpret_cast<float4*>(p);
-    const float4* z4 = reinterpret_cast<const float4*>(z);
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n4; i += (size_t)gridDim.x * blockDim.x) {
-        if (chunk && !chunk[i >> 10]) continue;
-        const float4 zi = z4[i];
-        float4 pi = p4[i];
-        pi.x = zi.x + b * pi.x; pi.y = zi.y + b * pi.y; pi.z = zi.z + b * pi.z; pi.w = zi.w + b * pi.w;
-        p4[i] = pi;
-    }
-}
-
-
 // p = z + b p
 template <typename T, typename TZ>
-__global__ void k_pcg_p(T* __restrict__ p, const TZ* __restrict__ z, double beta, size_t n) {
-    const T b = (T)beta;
+__global__ void k_pcg_p(T* __restrict__ p, const TZ* __restrict__ z, Coefs beta, size_t n) {
+    const T b = (T)beta.v[blockIdx.y];
+    p += blockIdx.y * n;
+    z += blockIdx.y * n;
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
         p[i] = (T)z[i] + b * p[i];
 }
 template <typename T, typename TZ>
-void launch_pcg_update_p(T* p, const TZ* z, double beta, size_t n, hipStream_t s, const uint8_t* chunk) {
-    if constexpr (std::is_same<T, float>::value && std::is_same<TZ, float>::value) {
-        if (n % 4 == 0) {
-            hipLaunchKernelGGL(k_pcg_p4, dim3(kStreamBlocks), dim3(256), 0, s, p, z, (float)beta, n / 4, chunk);
-            RT_HIP(hipGetLastError());
-            return;
-        }
-    }
-    unsigned nb = (unsigned)std::min<size_t>((n + 255) / 256, 16384);
-    hipLaunchKernelGGL((k_pcg_p<T, TZ>), dim3(nb), dim3(256), 0, s, p, z, beta, n);
+void launch_pcg_update_p(T* p, const TZ* z, Coefs beta, size_t n, hipStream_t s, int nb) {
+    unsigned blocks = (unsigned)std::min<size_t>((n + 255) / 256, 16384);
+    hipLaunchKernelGGL((k_pcg_p<T, TZ>), dim3(blocks, nb), dim3(256), 0, s, p, z, beta, n);
     RT_HIP(hipGetLastError());
 }
 
@@ -1267,9 +1258,9 @@ RT_INST_CS(float, bf16)
 
 #define RT_INST_T(T)                                                                                                  \
     template void launch_restrict<T>(const Geom&, const int*, Vec3<const T>, const Geom&, const int*, Vec3<T>,        \
-                                     const uint8_t*, int, T*, hipStream_t);                                           \
+                                     const uint8_t*, int, T*, hipStream_t, int);                                        \
     template void launch_prolong<T>(const Geom&, const int*, Vec3<T>, const uint8_t*, const Geom&, const int*,        \
-                                    Vec3<const T>, int, bool, hipStream_t);                                           \
+                                    Vec3<const T>, int, bool, hipStream_t, int);                                           \
     template void launch_coarsest<T>(const double*, int, const int*, Vec3<const T>, Vec3<T>, double*, hipStream_t);   \
     template void launch_fill<T>(T*, T, size_t, hipStream_t);                                                         \
     template void launch_box_to_oct<T>(const Geom&, const T*, T*, int, hipStream_t);                                  \
@@ -1285,15 +1276,15 @@ template void launch_convert<float, double>(const float*, double*, size_t, hipSt
 template void launch_convert<float, float>(const float*, float*, size_t, hipStream_t);
 template void launch_convert<double, double>(const double*, double*, size_t, hipStream_t);
 template void launch_dot_partials_t<double, double>(const double*, const double*, size_t, double*, int, hipStream_t,
-                                                  const uint8_t*);
+                                                  const uint8_t*, int, int);
 template void launch_dot_partials_t<double, float>(const double*, const float*, size_t, double*, int, hipStream_t,
-                                                  const uint8_t*);
+                                                  const uint8_t*, int, int);
 template void launch_dot_partials_t<float, float>(const float*, const float*, size_t, double*, int, hipStream_t,
-                                                  const uint8_t*);
+                                                  const uint8_t*, int, int);
 #define RT_INST_PCG(T, TZ)                                                                                        \
-    template void launch_pcg_update_x_r<T, TZ>(T*, T*, const T*, const T*, double, size_t, double*, int, TZ*,        \
-                                               hipStream_t);                                                       \
-    template void launch_pcg_update_p<T, TZ>(T*, const TZ*, double, size_t, hipStream_t, const uint8_t*);                          \
+    template void launch_pcg_update_x_r<T, TZ>(T*, T*, const T*, const T*, Coefs, size_t, double*, int, TZ*,         \
+                                               hipStream_t, int, int);                                             \
+    template void launch_pcg_update_p<T, TZ>(T*, const TZ*, Coefs, size_t, hipStream_t, int);                      \
     template void launch_sub_conv<T, TZ>(const T*, const T*, T*, TZ*, size_t, double*, int, hipStream_t);          \
     template void launch_add_conv<T, TZ>(T*, const TZ*, size_t, hipStream_t);
 RT_INST_PCG(double, float)

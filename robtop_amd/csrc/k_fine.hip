@@ -326,9 +326,11 @@ __device__ __forceinline__ double gs_blk_sum(double v) {
 template <typename T, int CY, int CZ, bool REV, bool ZS, bool Z0 = false, bool DOT = false>
 __global__ void __launch_bounds__(256) RT_GS_ATTR k_fine_gs_pair(Geom g, Vec3<T> U, Vec3<const T> F,
                                                       const float* __restrict__ rhop,
-                                                      const uint8_t* __restrict__ vflag, KeC<T> K, int nrows,
+                                                      const uint8_t* __restrict__ vflag, KeC<T> K, int nrows, int bs,
                                                       double* __restrict__ fu_part = nullptr) {
     static_assert(!(Z0 && REV), "a zero-start sweep runs forward");
+    at_batch(U, blockIdx.y, bs);
+    at_batch(F, blockIdx.y, bs);
     double fu = 0;
     double* fup = DOT ? &fu : nullptr;
     const int nhy = (g.n[1] - CY + 1) >> 1;
@@ -532,8 +534,10 @@ template <typename T> constexpr int kRowWaves = sizeof(T) == 4 ? 4 : 2;
 template <typename T, int CY, int CZ, bool REV, bool ZS, bool Z0 = false, bool DOT = false>
 __global__ void __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(kRowWaves<T>)))
 k_fine_gs_row(Geom g, Vec3<T> U, Vec3<const T> F, const float* __restrict__ rhop, const uint8_t* __restrict__ vflag,
-              KeC<T> K, int nrows, int rpw, int npr, double* __restrict__ fu_part) {
+              KeC<T> K, int nrows, int rpw, int npr, int bs, double* __restrict__ fu_part) {
     static_assert(!(Z0 && REV), "a zero-start sweep runs forward");
+    at_batch(U, blockIdx.y, bs);
+    at_batch(F, blockIdx.y, bs);
     constexpr int CE = (CY << 1) | (CZ << 2);
     __shared__ T sh[3][kRowThreads];         // new values of the parity relaxed first
     const int nhy = (g.n[1] - CY + 1) >> 1;
@@ -877,7 +881,7 @@ template void launch_fine_gs_sweep2<float>(const Geom&, Vec3<const float>, Vec3<
 template void launch_fine_gs_sweep2<double>(const Geom&, Vec3<const double>, Vec3<double>, Vec3<const double>,
                                             const float*, const uint8_t*, bool, bool, hipStream_t);
 
-// the row kernel's workgroup for a launch of `rows` rows: rpw whole rows (0: too
+// the row kernel's workgroup for a launch of `rows` rows (of all its vectors): rpw whole rows (0: too
 // long for it) of npr pairs in nt threads. Boxes are a multiple of the coarsest
 // spacing plus one node long, so a row's pairs often pass a multiple of 64 by
 // one. Where a launch fills the chip, the last pair's thread then takes the
@@ -921,26 +925,27 @@ int fine_gs_pair_blocks(const Geom& g, int pair) {
 
 template <typename T>
 void launch_fine_gs(const Geom& g, Vec3<T> U, Vec3<const T> F, const float* rhop, const uint8_t* vflag, int pair,
-                    bool reverse, bool zero_support, hipStream_t s, bool zero_start, double* fu_part) {
+                    bool reverse, bool zero_support, hipStream_t s, bool zero_start, double* fu_part, int nb) {
     check_buffer_range<T>(g);
     const int cy = pair & 1, cz = pair >> 1;
     const long long rows = (long long)((g.n[1] - cy + 1) >> 1) * ((g.n[2] - cz + 1) >> 1);
     if (rows <= 0) return;
-    if (fu_part && (!reverse || !zero_support || zero_start))
+    if (fu_part && (!reverse || !zero_support || zero_start || nb != 1))
         throw std::logic_error("f.u partials come from a reverse sweep with zero supports");
     if (zero_start && (reverse || !zero_support))
         throw std::logic_error("a zero-start sweep is forward with zero supports");
     const KeC<T> K = kec<T>();
-    const RowShape w = row_shape<T>(g, rows);
+    const RowShape w = row_shape<T>(g, rows * nb);
     const bool row = w.rpw > 0;
-    const dim3 grid(row ? (unsigned)((rows + w.rpw - 1) / w.rpw) : (unsigned)rows), block(row ? w.nt : 256);
+    const dim3 grid(row ? (unsigned)((rows + w.rpw - 1) / w.rpw) : (unsigned)rows, nb), block(row ? w.nt : 256);
+    const int bs = 3 * g.N;
 #define RT_LAUNCH(p, ...)                                                                                            \
     if (row)                                                                                                         \
         hipLaunchKernelGGL((k_fine_gs_row<T, ((p) & 1), ((p) >> 1), __VA_ARGS__>), grid, block, 0, s, g, U, F, rhop, \
-                           vflag, K, (int)rows, w.rpw, w.npr, fu_part);                                              \
+                           vflag, K, (int)rows, w.rpw, w.npr, bs, fu_part);                                          \
     else                                                                                                             \
         hipLaunchKernelGGL((k_fine_gs_pair<T, ((p) & 1), ((p) >> 1), __VA_ARGS__>), grid, block, 0, s, g, U, F, rhop, \
-                           vflag, K, (int)rows, fu_part);                                                            \
+                           vflag, K, (int)rows, bs, fu_part);                                                        \
     break;
     switch (pair * 8 + (fu_part ? 4 : zero_start ? 5 : (reverse ? 2 : 0) + (zero_support ? 1 : 0))) {
 #define RT_CASE(p)                                          \
@@ -958,8 +963,8 @@ void launch_fine_gs(const Geom& g, Vec3<T> U, Vec3<const T> F, const float* rhop
 }
 
 template void launch_fine_gs<float>(const Geom&, Vec3<float>, Vec3<const float>, const float*, const uint8_t*, int,
-                                    bool, bool, hipStream_t, bool, double*);
+                                    bool, bool, hipStream_t, bool, double*, int);
 template void launch_fine_gs<double>(const Geom&, Vec3<double>, Vec3<const double>, const float*, const uint8_t*, int,
-                                     bool, bool, hipStream_t, bool, double*);
+                                     bool, bool, hipStream_t, bool, double*, int);
 
 }  // namespace rt

@@ -99,8 +99,14 @@ template <typename T, int MODE>
 __global__ void __launch_bounds__(256) k_fine_res_modal(Geom g, Vec3<const T> U, Vec3<const T> F, Vec3<T> R,
                                                         const float* __restrict__ rhop,
                                                         const uint8_t* __restrict__ vflag, ModalK<T> K,
-                                                        double* __restrict__ partials) {
+                                                        double* __restrict__ partials, int gz, int bs, int pstride) {
     constexpr bool APPLY = MODE != 0;
+    // vector of a batch: the z blocks are gz per vector
+    const int bv = blockIdx.z / gz;
+    at_batch(U, bv, bs);
+    at_batch(F, bv, bs);
+    at_batch(R, bv, bs);
+    if (APPLY && partials) partials += (size_t)bv * pstride;
     __shared__ T su[2][3][PLANE];
     __shared__ uint8_t sf[2][PLANE];
     __shared__ T sy[24][256];
@@ -111,8 +117,8 @@ __global__ void __launch_bounds__(256) k_fine_res_modal(Geom g, Vec3<const T> U,
     // each XCD marches one contiguous range of tiles (x fastest), so the tiles
     // that share halo rows and partly used cache lines meet in one L2.
     const int gx = gridDim.x, gy = gridDim.y;
-    const int bl = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
-    const int bm = RT_MODAL_XCD ? xcd_row(bl, gx * gy * (int)gridDim.z) : bl;
+    const int bl = blockIdx.x + gx * (blockIdx.y + gy * (blockIdx.z - bv * gz));
+    const int bm = RT_MODAL_XCD ? xcd_row(bl, gx * gy * gz) : bl;
     if (g.tile_act && !g.tile_act[bm]) {   // no active node in this tile: nothing to write
         if (APPLY && partials && tid == 0) partials[bl] = 0.0;
         return;
@@ -316,28 +322,34 @@ int fine_apply_partials_modal(const Geom& g) {
 
 template <typename T>
 void launch_fine_residual_modal(const Geom& g, Vec3<const T> U, Vec3<const T> F, Vec3<T> R, const float* rhop,
-                                const uint8_t* vflag, hipStream_t s) {
-    hipLaunchKernelGGL((k_fine_res_modal<T, 0>), modal_grid(g), dim3(256), 0, s, g, U, F, R, rhop, vflag,
-                       modal_values<T>(g_modal), (double*)nullptr);
+                                const uint8_t* vflag, hipStream_t s, int nb) {
+    dim3 grid = modal_grid(g);
+    const int gz = (int)grid.z;
+    grid.z *= nb;
+    hipLaunchKernelGGL((k_fine_res_modal<T, 0>), grid, dim3(256), 0, s, g, U, F, R, rhop, vflag,
+                       modal_values<T>(g_modal), (double*)nullptr, gz, 3 * g.N, 0);
     RT_HIP(hipGetLastError());
 }
 
 template <typename T>
 void launch_fine_apply_modal(const Geom& g, Vec3<const T> X, Vec3<T> Y, const float* rhop, const uint8_t* vflag,
-                             double* partials, int* nparts, hipStream_t s) {
-    hipLaunchKernelGGL((k_fine_res_modal<T, 1>), modal_grid(g), dim3(256), 0, s, g, X, X, Y, rhop, vflag,
-                       modal_values<T>(g_modal), partials);
+                             double* partials, int* nparts, hipStream_t s, int nb, int pstride) {
+    dim3 grid = modal_grid(g);
+    const int gz = (int)grid.z;
+    grid.z *= nb;
+    hipLaunchKernelGGL((k_fine_res_modal<T, 1>), grid, dim3(256), 0, s, g, X, X, Y, rhop, vflag,
+                       modal_values<T>(g_modal), partials, gz, 3 * g.N, pstride);
     RT_HIP(hipGetLastError());
     if (nparts) *nparts = fine_apply_partials_modal(g);
 }
 
 template void launch_fine_residual_modal<float>(const Geom&, Vec3<const float>, Vec3<const float>, Vec3<float>,
-                                                const float*, const uint8_t*, hipStream_t);
+                                                const float*, const uint8_t*, hipStream_t, int);
 template void launch_fine_residual_modal<double>(const Geom&, Vec3<const double>, Vec3<const double>, Vec3<double>,
-                                                 const float*, const uint8_t*, hipStream_t);
+                                                 const float*, const uint8_t*, hipStream_t, int);
 template void launch_fine_apply_modal<float>(const Geom&, Vec3<const float>, Vec3<float>, const float*, const uint8_t*,
-                                             double*, int*, hipStream_t);
+                                             double*, int*, hipStream_t, int, int);
 template void launch_fine_apply_modal<double>(const Geom&, Vec3<const double>, Vec3<double>, const float*,
-                                              const uint8_t*, double*, int*, hipStream_t);
+                                              const uint8_t*, double*, int*, hipStream_t, int, int);
 
 }  // namespace rt

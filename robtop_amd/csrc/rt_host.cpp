@@ -618,23 +618,24 @@ static void residual(Hier& H, int li, Vec3<const T> U, Vec3<const T> F, Vec3<T> 
 }
 
 template <typename T>
-static void restrict_to(Hier& H, int li, Vec3<const T> Rf, Vec3<T> Fc) {
+static void restrict_to(Hier& H, int li, Vec3<const T> Rf, Vec3<T> Fc, int nb = 1) {
     Level& C = H.lv[li];
     Level& Fl = H.lv[li - 1];
     const int ratio = C.scale / Fl.scale;
     T* scratch = nullptr;
-    if (ratio == 4 && H.xfer.bytes >= sizeof(T) * restrict_scratch_elems(Fl.g, C.g)) scratch = H.xfer.as<T>();
-    launch_restrict<T>(Fl.g, Fl.o, Rf, C.g, C.o, Fc, C.vflag.as<uint8_t>(), ratio, scratch, H.s);
+    if (ratio == 4 && H.xfer.bytes >= sizeof(T) * nb * restrict_scratch_elems(Fl.g, C.g)) scratch = H.xfer.as<T>();
+    launch_restrict<T>(Fl.g, Fl.o, Rf, C.g, C.o, Fc, C.vflag.as<uint8_t>(), ratio, scratch, H.s, nb);
 }
 
 template <typename T>
 // skip_fixed leaves support nodes untouched; the smoother that follows resets
 // them to f / n_e and their neighbours ignore them, so the cycle's result is
 // the same either way (Grid.cu:1818-1895 corrects them too)
-static void prolong_from(Hier& H, int li, Vec3<T> Uf, Vec3<const T> Uc, bool skip_fixed = false) {
+static void prolong_from(Hier& H, int li, Vec3<T> Uf, Vec3<const T> Uc, bool skip_fixed = false, int nb = 1) {
     Level& Fl = H.lv[li];
     Level& C = H.lv[li + 1];
-    launch_prolong<T>(Fl.g, Fl.o, Uf, Fl.vflag.as<uint8_t>(), C.g, C.o, Uc, C.scale / Fl.scale, skip_fixed, H.s);
+    launch_prolong<T>(Fl.g, Fl.o, Uf, Fl.vflag.as<uint8_t>(), C.g, C.o, Uc, C.scale / Fl.scale, skip_fixed, H.s,
+                      nb);
 }
 
 template <typename T>
@@ -1404,8 +1405,7 @@ static void pcg_reliable(Hier& H, double tol, int maxit, int pre, int post, rt_s
             if (!(pq > 0)) throw std::domain_error("PCG breakdown: p.Ap <= 0");
             const double alpha = rz / pq;
             H.cg_alpha.push_back(alpha);
-            launch_pcg_ru_dxr(pc.F.data(), H.q32.data(), nullptr, nullptr, alpha, n, H.partials.as<double>(), ns,
-                              H.s, vec_chunks(H));
+            launch_pcg_ru_r(pc.F.data(), H.q32.data(), alpha, n, H.partials.as<double>(), ns, H.s, vec_chunks(H));
             apend = alpha;
             flushed = false;
             const double rn = std::sqrt(sum_partials_host(H, ns));
@@ -1428,10 +1428,7 @@ static void pcg_reliable(Hier& H, double tol, int maxit, int pre, int post, rt_s
             const double beta = rz_new / rz;
             H.cg_beta.push_back(beta);
             rz = rz_new;
-            if (apend != 0.0)
-                launch_pcg_p_dx(H.p32.data(), pc.U.data(), beta, H.dx32.data(), apend, n, H.s, vec_chunks(H));
-            else
-                launch_pcg_update_p<float, float>(H.p32.data(), pc.U.data(), beta, n, H.s, vec_chunks(H));
+            launch_pcg_p_dx(H.p32.data(), pc.U.data(), beta, H.dx32.data(), apend, n, H.s, vec_chunks(H));
             apend = 0.0;
         }
         if (!flushed) launch_pcg_flush_x(H.x64.data(), H.dx32.data(), n, H.s, H.p32.data(), apend);
@@ -2703,12 +2700,15 @@ static void worst_apply(Hier& H, const double* q, double* y, double solve_tol, i
 
 // ---------------------------------------------------------------------------
 // Batched solves for the worst-case search: nb <= kBatchMax right-hand sides
-// through one preconditioner cycle. The finest level (whose traffic is the
-// vectors themselves) runs the single-vector kernels once per vector; every
-// coarser level runs batched kernels that read each stencil coefficient once
-// for all nb vectors, and the coarsest applies its inverse to all nb at once.
-// The whole batched cycle is captured into one HIP graph. No counterpart in
-// the reference, which solves one load at a time (optimization.cpp:123-261).
+// through one preconditioner cycle. Every kernel of the cycle and of the CG
+// takes all vectors in one launch: a vector of a small or middling grid does not
+// fill the chip by itself, and the launches of eight cost eight times their
+// latency (block Lanczos on a 128^3 torus: 155 ms with the finest level's and the
+// CG's kernels launched per vector, 99 ms so). The coarser levels read each
+// stencil coefficient once for all nb vectors, and the coarsest applies its
+// inverse to all nb at once. The whole batched cycle is captured into one HIP
+// graph. No counterpart in the reference, which solves one load at a time
+// (optimization.cpp:123-261).
 // ---------------------------------------------------------------------------
 static bool batch_supported(const Hier& H) { return H.pc_gamma == 1 && H.coarse_bits == 32; }
 
@@ -2733,6 +2733,15 @@ static void ensure_batch(Hier& H, int nb) {
     H.bfbuf.ensure(sizeof(double) * (size_t)nb * std::max(std::max(H.n3, H.pcn3), 1));
     for (BVec<float>* v : {&H.bp32, &H.bq32, &H.bdx32})
         if (!v->fits(N, nb)) { v->alloc(N, nb); grown = true; }
+    // the x4 restriction's scratch, per vector; a captured cycle holds its address
+    for (size_t li = 1; li < H.lv.size(); li++)
+        if (H.lv[li].scale / H.lv[li - 1].scale == 4) {
+            const size_t need = sizeof(float) * nb * restrict_scratch_elems(H.lv[li - 1].g, H.lv[li].g);
+            if (H.xfer.bytes < need) {
+                H.drop_graph();
+                H.xfer.ensure(need);
+            }
+        }
     H.bpart.ensure(sizeof(double) * (size_t)nb * batch_part_stride(H));
     H.bscal.ensure(sizeof(double) * kBatchMax);
     if (grown && H.bgraph) {
@@ -2750,8 +2759,15 @@ static void vcycle_batch(Hier& H, int nb, int pre, int post) {
     // zero_start: the fine vectors hold no valid values yet (first pre-smoothing)
     auto smooth = [&](int i, int nsw, bool rev, bool zero_start) {
         Level& L = H.lv[i];
-        if (i == 0) {
+        if (i == 0 && (H.fine_smoother == 1 || nsw == 0)) {
             for (int b = 0; b < nb; b++) gs<float>(H, 0, L.bU.v(b), L.bF.cv(b), nsw, rev, true, zero_start);
+            return;
+        }
+        if (i == 0) {
+            for (int it = 0; it < nsw; it++)
+                for (int pp = 0; pp < 4; pp++)
+                    launch_fine_gs<float>(L.g, L.bU.v(0), L.bF.cv(0), H.rhop.as<float>(), L.vflag.as<uint8_t>(),
+                                          rev ? 3 - pp : pp, rev, true, H.s, zero_start && it == 0, nullptr, nb);
             return;
         }
         for (int it = 0; it < nsw; it++)
@@ -2770,15 +2786,16 @@ static void vcycle_batch(Hier& H, int nb, int pre, int post) {
         const int m = i == 0 ? 1 : level_mult(H, i);
         smooth(i, pre * m, false, i == 0);
         if (i == 0)
-            for (int b = 0; b < nb; b++) residual<float>(H, 0, L.bU.cv(b), L.bF.cv(b), L.bR.v(b));
+            launch_fine_residual_modal<float>(L.g, L.bU.cv(0), L.bF.cv(0), L.bR.v(0), H.rhop.as<float>(),
+                                              L.vflag.as<uint8_t>(), H.s, nb);
         else
             launch_coarse_residual_batch<float, float>(L.g, nb, L.bU.data(), L.bF.data(), L.bR.data(),
                                                        L.st32.as<float>(), L.vflag.as<uint8_t>(), H.s);
         Level& C = H.lv[i + 1];
-        for (int b = 0; b < nb; b++) restrict_to<float>(H, i + 1, L.bR.cv(b), C.bF.v(b));
+        restrict_to<float>(H, i + 1, L.bR.cv(0), C.bF.v(0), nb);
         launch_fill<float>(C.bU.data(), 0.f, (size_t)3 * C.g.N * nb, H.s);
         self(self, i + 1);
-        for (int b = 0; b < nb; b++) prolong_from<float>(H, i, L.bU.v(b), C.bU.cv(b), i == 0);
+        prolong_from<float>(H, i, L.bU.v(0), C.bU.cv(0), i == 0, nb);
         if (i == 0)
             for (int b = 0; b < nb; b++)
                 island_correct<float>(L.g, H.nisl, H.isl_nodes, H.isl_cnt.as<int>(), H.isl_node.as<int>(),
@@ -2823,10 +2840,20 @@ static void precondition_batch(Hier& H, int nb, int pre, int post) {
 
 // out[b] = sum of the np partials of vector b (bpart + b * stride), one sync
 static void batch_sums(Hier& H, int nb, int np, int stride, double* out) {
-    for (int b = 0; b < nb; b++)
-        launch_sum_partials(H.bpart.as<double>() + (size_t)b * stride, np, H.bscal.as<double>() + b, H.s);
+    launch_sum_partials(H.bpart.as<double>(), np, H.bscal.as<double>(), H.s, nb, stride);
     RT_HIP(hipMemcpyAsync(out, H.bscal.p, sizeof(double) * nb, hipMemcpyDeviceToHost, H.s));
     RT_HIP(hipStreamSynchronize(H.s));
+}
+
+// f(b, n) for every run of n flagged vectors from b on: one launch each
+template <typename F>
+static void active_runs(const bool* act, int nb, F&& f) {
+    for (int b = 0; b < nb;) {
+        int e = b;
+        while (e < nb && act[e]) e++;
+        if (e > b) f(b, e - b);
+        b = e + 1;
+    }
 }
 
 // nb preconditioned CG solves K x_b = f_b (H.bb -> H.bx, from zero) in
@@ -2839,16 +2866,14 @@ static void pcg_batch(Hier& H, int nb, double tol, int maxit, int pre, int post,
     Level& L0 = H.lv[0];
     const size_t n = (size_t)3 * L0.g.N;
     const int np = 1024, npa = batch_part_stride(H);
-    double nf[kBatchMax], rr[kBatchMax], rz[kBatchMax], pq[kBatchMax];
+    double nf[kBatchMax], rr[kBatchMax], rz[kBatchMax], pq[kBatchMax], c[kBatchMax] = {};
+    double* part = H.bpart.as<double>();
     bool act[kBatchMax];
-    for (int b = 0; b < nb; b++) {
-        launch_fill<double>(H.bx.at(b), 0.0, n, H.s);
-        launch_convert<double, double>(H.bb.at(b), H.br.at(b), n, H.s);
-        launch_convert<double, float>(H.bb.at(b), L0.bF.at(b), n, H.s);
-        launch_dot_partials_t<double, double>(H.bb.at(b), H.bb.at(b), n, H.bpart.as<double>() + (size_t)b * npa, np,
-                                              H.s);
-        iters[b] = 0;
-    }
+    launch_fill<double>(H.bx.data(), 0.0, n * nb, H.s);
+    launch_convert<double, double>(H.bb.data(), H.br.data(), n * nb, H.s);
+    launch_convert<double, float>(H.bb.data(), L0.bF.data(), n * nb, H.s);
+    launch_dot_partials_t<double, double>(H.bb.data(), H.bb.data(), n, part, np, H.s, nullptr, nb, npa);
+    for (int b = 0; b < nb; b++) iters[b] = 0;
     batch_sums(H, nb, np, npa, nf);
     int live = 0;
     for (int b = 0; b < nb; b++) {
@@ -2858,27 +2883,26 @@ static void pcg_batch(Hier& H, int nb, double tol, int maxit, int pre, int post,
     }
     if (live) {
         precondition_batch(H, nb, pre, post);
-        for (int b = 0; b < nb; b++) {
-            launch_dot_partials_t<double, float>(H.br.at(b), L0.bU.at(b), n, H.bpart.as<double>() + (size_t)b * npa,
-                                                 np, H.s);
-            launch_convert<float, double>(L0.bU.at(b), H.bp.at(b), n, H.s);
-        }
+        launch_dot_partials_t<double, float>(H.br.data(), L0.bU.data(), n, part, np, H.s, nullptr, nb, npa);
+        launch_convert<float, double>(L0.bU.data(), H.bp.data(), n * nb, H.s);
         batch_sums(H, nb, np, npa, rz);
     }
     for (int it = 1; it <= maxit && live; it++) {
         int npq = 0;
-        for (int b = 0; b < nb; b++) {
-            if (!act[b]) continue;
+        active_runs(act, nb, [&](int b, int k) {
             launch_fine_apply_modal<double>(L0.g, H.bp.cv(b), H.bq.v(b), H.rhop.as<float>(), L0.vflag.as<uint8_t>(),
-                                            H.bpart.as<double>() + (size_t)b * npa, &npq, H.s);
-        }
+                                            part + (size_t)b * npa, &npq, H.s, k, npa);
+        });
         batch_sums(H, nb, npq, npa, pq);
         for (int b = 0; b < nb; b++) {
             if (!act[b]) continue;
             if (!(pq[b] > 0)) throw std::domain_error("PCG breakdown: p.Ap <= 0");
-            launch_pcg_update_x_r<double, float>(H.bx.at(b), H.br.at(b), H.bp.at(b), H.bq.at(b), rz[b] / pq[b], n,
-                                                 H.bpart.as<double>() + (size_t)b * npa, np, L0.bF.at(b), H.s);
+            c[b] = rz[b] / pq[b];
         }
+        active_runs(act, nb, [&](int b, int k) {
+            launch_pcg_update_x_r<double, float>(H.bx.at(b), H.br.at(b), H.bp.at(b), H.bq.at(b), Coefs(c + b, k), n,
+                                                 part + (size_t)b * npa, np, L0.bF.at(b), H.s, k, npa);
+        });
         batch_sums(H, nb, np, npa, rr);
         live = 0;
         for (int b = 0; b < nb; b++) {
@@ -2889,25 +2913,27 @@ static void pcg_batch(Hier& H, int nb, double tol, int maxit, int pre, int post,
         }
         if (!live) break;
         precondition_batch(H, nb, pre, post);
-        for (int b = 0; b < nb; b++)
-            if (act[b])
-                launch_dot_partials_t<double, float>(H.br.at(b), L0.bU.at(b), n,
-                                                     H.bpart.as<double>() + (size_t)b * npa, np, H.s);
+        active_runs(act, nb, [&](int b, int k) {
+            launch_dot_partials_t<double, float>(H.br.at(b), L0.bU.at(b), n, part + (size_t)b * npa, np, H.s, nullptr, k,
+                                                 npa);
+        });
         double rzn[kBatchMax];
         batch_sums(H, nb, np, npa, rzn);
         for (int b = 0; b < nb; b++) {
             if (!act[b]) continue;
-            launch_pcg_update_p<double, float>(H.bp.at(b), L0.bU.at(b), rzn[b] / rz[b], n, H.s);
+            c[b] = rzn[b] / rz[b];
             rz[b] = rzn[b];
         }
+        active_runs(act, nb, [&](int b, int k) {
+            launch_pcg_update_p<double, float>(H.bp.at(b), L0.bU.at(b), Coefs(c + b, k), n, H.s, k);
+        });
     }
     // true residuals |f_b - K x_b| / |f_b|
-    for (int b = 0; b < nb; b++) {
-        launch_fine_apply_modal<double>(L0.g, H.bx.cv(b), H.bq.v(b), H.rhop.as<float>(), L0.vflag.as<uint8_t>(),
-                                        nullptr, nullptr, H.s);
+    launch_fine_apply_modal<double>(L0.g, H.bx.cv(0), H.bq.v(0), H.rhop.as<float>(), L0.vflag.as<uint8_t>(), nullptr,
+                                    nullptr, H.s, nb);
+    for (int b = 0; b < nb; b++)
         launch_sub_conv<double, double>(H.bb.at(b), H.bq.at(b), H.br.at(b), (double*)nullptr, n,
-                                        H.bpart.as<double>() + (size_t)b * npa, np, H.s);
-    }
+                                        part + (size_t)b * npa, np, H.s);
     batch_sums(H, nb, np, npa, rr);
     for (int b = 0; b < nb; b++) rel[b] = nf[b] > 0 ? std::sqrt(rr[b]) / nf[b] : 0.0;
 }
@@ -2931,12 +2957,12 @@ static void pcg_batch_reliable(Hier& H, int nb, double tol, int maxit, int pre, 
     bool act[kBatchMax], bad[kBatchMax], dirty[kBatchMax];
     // apend[b]: the step whose alpha p is not yet on dx (added by the next
     // direction update or by the flush, as in pcg_reliable)
-    double apend[kBatchMax] = {};
+    double apend[kBatchMax] = {}, c[kBatchMax] = {};
+    launch_fill<double>(H.bx.data(), 0.0, n * nb, H.s);
+    launch_fill<float>(H.bdx32.data(), 0.f, n * nb, H.s);
+    launch_convert<double, float>(H.bb.data(), L0.bF.data(), n * nb, H.s);
+    launch_dot_partials_t<double, double>(H.bb.data(), H.bb.data(), n, part, np, H.s, nullptr, nb, npa);
     for (int b = 0; b < nb; b++) {
-        launch_fill<double>(H.bx.at(b), 0.0, n, H.s);
-        launch_fill<float>(H.bdx32.at(b), 0.f, n, H.s);
-        launch_convert<double, float>(H.bb.at(b), L0.bF.at(b), n, H.s);
-        launch_dot_partials_t<double, double>(H.bb.at(b), H.bb.at(b), n, part + (size_t)b * npa, np, H.s);
         iters[b] = 0;
         bad[b] = dirty[b] = false;
     }
@@ -2952,10 +2978,12 @@ static void pcg_batch_reliable(Hier& H, int nb, double tol, int maxit, int pre, 
     }
     // true residuals of the vectors in `which`: r64 = f - K x64, rt[b] = |r64| / |f|
     auto true_res = [&](const bool* which) {
+        active_runs(which, nb, [&](int b, int k) {
+            launch_fine_apply_modal<double>(L0.g, H.bx.cv(b), H.bq.v(b), H.rhop.as<float>(), L0.vflag.as<uint8_t>(),
+                                            nullptr, nullptr, H.s, k);
+        });
         for (int b = 0; b < nb; b++) {
             if (!which[b]) continue;
-            launch_fine_apply_modal<double>(L0.g, H.bx.cv(b), H.bq.v(b), H.rhop.as<float>(), L0.vflag.as<uint8_t>(),
-                                            nullptr, nullptr, H.s);
             launch_sub_conv<double, double>(H.bb.at(b), H.bq.at(b), H.br.at(b), (double*)nullptr, n,
                                             part + (size_t)b * npa, np, H.s);
         }
@@ -2966,28 +2994,27 @@ static void pcg_batch_reliable(Hier& H, int nb, double tol, int maxit, int pre, 
     };
     if (live) {
         precondition_batch(H, nb, pre, post);
-        for (int b = 0; b < nb; b++) {
-            launch_dot_partials_t<float, float>(L0.bF.at(b), L0.bU.at(b), n, part + (size_t)b * npa, ns, H.s,
-                                                vec_chunks(H));
-            launch_convert<float, float>(L0.bU.at(b), H.bp32.at(b), n, H.s);
-        }
+        launch_dot_partials_t<float, float>(L0.bF.data(), L0.bU.data(), n, part, ns, H.s, vec_chunks(H), nb, npa);
+        launch_convert<float, float>(L0.bU.data(), H.bp32.data(), n * nb, H.s);
         batch_sums(H, nb, ns, npa, rz);
     }
     for (int it = 1; it <= maxit && live; it++) {
         int npq = 0;
-        for (int b = 0; b < nb; b++)
-            if (act[b])
-                launch_fine_apply_modal<float>(L0.g, H.bp32.cv(b), H.bq32.v(b), H.rhop.as<float>(),
-                                               L0.vflag.as<uint8_t>(), part + (size_t)b * npa, &npq, H.s);
+        active_runs(act, nb, [&](int b, int k) {
+            launch_fine_apply_modal<float>(L0.g, H.bp32.cv(b), H.bq32.v(b), H.rhop.as<float>(),
+                                           L0.vflag.as<uint8_t>(), part + (size_t)b * npa, &npq, H.s, k, npa);
+        });
         batch_sums(H, nb, npq, npa, pq);
         for (int b = 0; b < nb; b++) {
             if (!act[b]) continue;
             if (!(pq[b] > 0)) throw std::domain_error("PCG breakdown: p.Ap <= 0");
             apend[b] = rz[b] / pq[b];
-            launch_pcg_ru_dxr(L0.bF.at(b), H.bq32.at(b), nullptr, nullptr, apend[b], n, part + (size_t)b * npa, ns,
-                              H.s, vec_chunks(H));
             dirty[b] = true;
         }
+        active_runs(act, nb, [&](int b, int k) {
+            launch_pcg_ru_r(L0.bF.at(b), H.bq32.at(b), Coefs(apend + b, k), n, part + (size_t)b * npa, ns, H.s,
+                            vec_chunks(H), k, npa);
+        });
         batch_sums(H, nb, ns, npa, rn);
         bool rep[kBatchMax] = {};
         int nrep = 0;
@@ -3019,19 +3046,20 @@ static void pcg_batch_reliable(Hier& H, int nb, double tol, int maxit, int pre, 
         for (int b = 0; b < nb; b++) live += act[b];
         if (!live) break;
         precondition_batch(H, nb, pre, post);
-        for (int b = 0; b < nb; b++)
-            if (act[b])
-                launch_dot_partials_t<float, float>(L0.bF.at(b), L0.bU.at(b), n, part + (size_t)b * npa, ns, H.s,
-                                                    vec_chunks(H));
+        active_runs(act, nb, [&](int b, int k) {
+            launch_dot_partials_t<float, float>(L0.bF.at(b), L0.bU.at(b), n, part + (size_t)b * npa, ns, H.s,
+                                                vec_chunks(H), k, npa);
+        });
         double rzn[kBatchMax];
         batch_sums(H, nb, ns, npa, rzn);
+        for (int b = 0; b < nb; b++)
+            if (act[b]) c[b] = rzn[b] / rz[b];
+        active_runs(act, nb, [&](int b, int k) {
+            launch_pcg_p_dx(H.bp32.at(b), L0.bU.at(b), Coefs(c + b, k), H.bdx32.at(b), Coefs(apend + b, k), n, H.s,
+                            vec_chunks(H), k);
+        });
         for (int b = 0; b < nb; b++) {
             if (!act[b]) continue;
-            if (apend[b] != 0.0)
-                launch_pcg_p_dx(H.bp32.at(b), L0.bU.at(b), rzn[b] / rz[b], H.bdx32.at(b), apend[b], n, H.s,
-                                vec_chunks(H));
-            else
-                launch_pcg_update_p<float, float>(H.bp32.at(b), L0.bU.at(b), rzn[b] / rz[b], n, H.s, vec_chunks(H));
             apend[b] = 0.0;
             rz[b] = rzn[b];
         }

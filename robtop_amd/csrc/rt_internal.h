@@ -67,6 +67,11 @@ __host__ __device__ inline int oct_index(const Geom& g, int qx, int qy, int qz) 
 __host__ __device__ inline int oct_p(const Geom& g, int x, int y, int z) { return oct_index(g, x + 2, y + 2, z + 2); }
 
 template <typename T> struct Vec3 { T* c[3]; };
+// vector b of a batch whose vectors lie bs values apart
+template <typename T> __device__ __forceinline__ void at_batch(Vec3<T>& v, unsigned b, int bs) {
+    const size_t o = (size_t)b * (size_t)bs;
+    v.c[0] += o; v.c[1] += o; v.c[2] += o;
+}
 
 // Workgroups are handed to the 8 XCDs round-robin (workgroup b runs on XCD
 // b % 8), and each XCD has its own L2. This maps workgroup b to a work index
@@ -110,6 +115,8 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* p, int bytes)
 // ---------------------------------------------------------------------------
 // kernel launchers (defined in the .hip files); all launch on stream `s`
 // ---------------------------------------------------------------------------
+// nb (where a launcher has it): the same on nb vectors in one launch, vector b
+// at + b 3N of its base (partials at + b pstride)
 // k_fine.hip
 void set_ke_constants(const double* ke576, hipStream_t s);
 // zero_start: the first forward sweep of a cycle from u = 0 with zero supports;
@@ -119,7 +126,7 @@ void set_ke_constants(const double* ke576, hipStream_t s);
 template <typename T>
 void launch_fine_gs(const Geom& g, Vec3<T> U, Vec3<const T> F, const float* rhop, const uint8_t* vflag, int pair,
                     bool reverse, bool zero_support, hipStream_t s, bool zero_start = false,
-                    double* fu_part = nullptr);
+                    double* fu_part = nullptr, int nb = 1);
 int fine_gs_pair_blocks(const Geom& g, int pair);   // FP32
 // one full fine sweep in two launches, old values from Uin, new ones to Uout
 // (Uin is not written; the two must not overlap)
@@ -131,10 +138,10 @@ void launch_fine_gs_sweep2(const Geom& g, Vec3<const T> Uin, Vec3<T> Uout, Vec3<
 void set_modal_constants(const double* ke576);
 template <typename T>
 void launch_fine_residual_modal(const Geom& g, Vec3<const T> U, Vec3<const T> F, Vec3<T> R, const float* rhop,
-                                const uint8_t* vflag, hipStream_t s);
+                                const uint8_t* vflag, hipStream_t s, int nb = 1);
 template <typename T>
 void launch_fine_apply_modal(const Geom& g, Vec3<const T> X, Vec3<T> Y, const float* rhop, const uint8_t* vflag,
-                             double* partials, int* nparts, hipStream_t s);
+                             double* partials, int* nparts, hipStream_t s, int nb = 1, int pstride = 0);
 int fine_apply_partials_modal(const Geom& g);
 // node tile of the residual / apply kernels (x by y; z by Geom::zc)
 void modal_tile_dims(int* tx, int* ty);
@@ -153,7 +160,6 @@ template <typename T, typename TS>
 void launch_coarse_residual(const Geom& g, Vec3<const T> U, Vec3<const T> F, Vec3<T> R, const TS* st,
                             const uint8_t* vflag, hipStream_t s);
 // batched coarse-level kernels: nb <= kBatchMax vectors, vector b at base + b 3N
-constexpr int kBatchMax = 8;
 template <typename T, typename TS>
 void launch_coarse_gs_batch(const Geom& g, int nb, T* U, const T* F, const TS* st, const uint8_t* vflag, int colour,
                             bool reverse, hipStream_t s);
@@ -166,12 +172,12 @@ void launch_coarsest_batch(const double* Ainv, int n3, const int* rowslot, int n
                            double* fbuf, hipStream_t s);
 template <typename T>
 void launch_restrict(const Geom& gf, const int of[3], Vec3<const T> Rf, const Geom& gc, const int oc[3], Vec3<T> Fc,
-                     const uint8_t* vflag_c, int ratio, T* scratch, hipStream_t s);
-// elements of T the two-stage x4 restriction needs as scratch
+                     const uint8_t* vflag_c, int ratio, T* scratch, hipStream_t s, int nb = 1);
+// elements of T the two-stage x4 restriction needs as scratch, per vector
 size_t restrict_scratch_elems(const Geom& gf, const Geom& gc);
 template <typename T>
 void launch_prolong(const Geom& gf, const int of[3], Vec3<T> Uf, const uint8_t* vflag_f, const Geom& gc,
-                    const int oc[3], Vec3<const T> Uc, int ratio, bool skip_fixed, hipStream_t s);
+                    const int oc[3], Vec3<const T> Uc, int ratio, bool skip_fixed, hipStream_t s, int nb = 1);
 template <typename T>
 void launch_coarsest(const double* Ainv, int n3, const int* rowslot, Vec3<const T> F, Vec3<T> U, double* fbuf,
                      hipStream_t s);
@@ -211,22 +217,29 @@ void launch_convert(const TA* a, TB* b, size_t n, hipStream_t s);
 template <typename T>
 void launch_fill(T* a, T v, size_t n, hipStream_t s);
 void launch_dot_partials(const double* a, const double* b, size_t n, double* partials, int nparts, hipStream_t s);
+// one coefficient per vector of a batch
+constexpr int kBatchMax = 8;
+struct Coefs {
+    double v[kBatchMax];
+    Coefs() = default;
+    Coefs(double x) : v{x} {}
+    explicit Coefs(const double* x, int n) : v{} { for (int i = 0; i < n; i++) v[i] = x[i]; }
+};
 template <typename TA, typename TB>
 void launch_dot_partials_t(const TA* a, const TB* b, size_t n, double* partials, int nparts, hipStream_t s,
-                           const uint8_t* chunk = nullptr);
-void launch_sum_partials(const double* partials, int nparts, double* out, hipStream_t s);
+                           const uint8_t* chunk = nullptr, int nb = 1, int pstride = 0);
+void launch_sum_partials(const double* partials, int nparts, double* out, hipStream_t s, int nb = 1, int pstride = 0);
 template <typename T, typename TZ>
-void launch_pcg_update_x_r(T* x, T* r, const T* p, const T* q, double alpha, size_t n, double* partials, int nparts,
-                           TZ* rz_out, hipStream_t s);
-// reliable-update PCG (FP32 vectors): r -= alpha q with partials of r.r, and
-// dx += alpha p unless dx is null
-void launch_pcg_ru_dxr(float* r, const float* q, float* dx, const float* p, double alpha, size_t n, double* partials,
-                       int nparts, hipStream_t s, const uint8_t* chunk = nullptr);
+void launch_pcg_update_x_r(T* x, T* r, const T* p, const T* q, Coefs alpha, size_t n, double* partials, int nparts,
+                           TZ* rz_out, hipStream_t s, int nb = 1, int pstride = 0);
+// reliable-update PCG (FP32 vectors, n a multiple of 4): r -= alpha q with partials of r.r
+void launch_pcg_ru_r(float* r, const float* q, Coefs alpha, size_t n, double* partials, int nparts, hipStream_t s,
+                     const uint8_t* chunk = nullptr, int nb = 1, int pstride = 0);
 // x64 += dx (+ alpha p, a pending increment, when p is given), dx = 0
 void launch_pcg_flush_x(double* x, float* dx, size_t n, hipStream_t s, const float* p = nullptr, double alpha = 0.0);
-// dx += alpha p, then p = z + beta p (FP32, n a multiple of 4)
-void launch_pcg_p_dx(float* p, const float* z, double beta, float* dx, double alpha, size_t n, hipStream_t s,
-                     const uint8_t* chunk = nullptr);
+// dx += alpha p (where alpha != 0), then p = z + beta p (FP32, n a multiple of 4)
+void launch_pcg_p_dx(float* p, const float* z, Coefs beta, float* dx, Coefs alpha, size_t n, hipStream_t s,
+                     const uint8_t* chunk = nullptr, int nb = 1);
 // streaming kernels' grid size (partials written by the reducing ones)
 #ifndef RT_STREAM_BLOCKS
 #define RT_STREAM_BLOCKS 2048
@@ -236,7 +249,7 @@ constexpr int kStreamBlocks = RT_STREAM_BLOCKS;
 // byte per 4096 floats: 0 where no active node's value lies)
 void launch_vec_chunks(const uint8_t* vflag, int N, uint8_t* chunk, hipStream_t s);
 template <typename T, typename TZ>
-void launch_pcg_update_p(T* p, const TZ* z, double beta, size_t n, hipStream_t s, const uint8_t* chunk = nullptr);
+void launch_pcg_update_p(T* p, const TZ* z, Coefs beta, size_t n, hipStream_t s, int nb = 1);
 template <typename T, typename TZ>
 void launch_sub_conv(const T* b, const T* q, T* r, TZ* rz, size_t n, double* partials, int nparts, hipStream_t s);
 template <typename T, typename TE>
