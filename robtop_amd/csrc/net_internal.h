@@ -39,6 +39,7 @@ size_t conv_wgrad_part_elems(int cin, int cout);
 // out[i] (+)= sum_w part[w][i], i < n
 void launch_sum_parts(const float* part, int nparts, size_t n, float* out, int accumulate, hipStream_t s);
 // bias gradient db[c] += sum_p G[p][c]
+constexpr int kBiasBlocks = 256;      // part: kBiasBlocks * c floats
 void launch_bias_grad(int c, size_t P, const uint16_t* G, float* part, float* db, hipStream_t s);
 // 2x2x2 average pool (windows clipped at the upper faces), nearest upsample,
 // and their transposes fused with the ReLU derivative
@@ -118,7 +119,7 @@ struct Net {
     size_t cap[3] = {0, 0, 0};              // positions the activations are sized for
     DBuf F, a0, s0, q1, a1, s1, q2, a2, b2, u1, c1, t1, u0, c0, t0, Y;
     DBuf gY, gt0, gc0, hu0, gt1, gc1, hu1, gb2, ga2, hq2, gs1, ga1, hq1, gs0, ga0;
-    DBuf wpart, bpart, lpart, T, absmax;
+    DBuf wpart, bpart, lpart, T, absmax, xin, yout;
     std::vector<NetSample*> samples;
     int adam_t = 0;
     ~Net();

@@ -74,7 +74,7 @@ static Net* net_new(uint64_t seed) {
         wp = std::max(wp, conv_wgrad_part_elems(kCin[l], kCout[l]));
     }
     N->wpart.alloc(sizeof(float) * wp);
-    N->bpart.alloc(sizeof(float) * 64 * 64);
+    N->bpart.alloc(sizeof(float) * kBiasBlocks * 64);
     N->lpart.alloc(sizeof(double) * kLossParts);
     N->absmax.alloc(sizeof(unsigned));
     std::vector<float> w;
@@ -353,14 +353,13 @@ int rt_net_forward(rt_net* n, const int* dims, const float* x, float* y) {
         Net& N = N_(n);
         shape(N, dims);
         const size_t P = P_of(dims);
-        DBuf xin, yout;
-        xin.alloc(sizeof(float) * P * 4);
-        yout.alloc(sizeof(float) * P * 3);
-        RT_HIP(hipMemcpyAsync(xin.p, x, sizeof(float) * P * 4, hipMemcpyHostToDevice, N.s));
-        launch_pack_input(P, xin.as<float>(), mb(N.F), N.s);
+        N.xin.ensure(sizeof(float) * P * 4);
+        N.yout.ensure(sizeof(float) * P * 3);
+        RT_HIP(hipMemcpyAsync(N.xin.p, x, sizeof(float) * P * 4, hipMemcpyHostToDevice, N.s));
+        launch_pack_input(P, N.xin.as<float>(), mb(N.F), N.s);
         forward(N, N.s);
-        launch_unpack_output(P, B<float>(N.Y), yout.as<float>(), N.s);
-        RT_HIP(hipMemcpyAsync(y, yout.p, sizeof(float) * P * 3, hipMemcpyDeviceToHost, N.s));
+        launch_unpack_output(P, B<float>(N.Y), N.yout.as<float>(), N.s);
+        RT_HIP(hipMemcpyAsync(y, N.yout.p, sizeof(float) * P * 3, hipMemcpyDeviceToHost, N.s));
         RT_HIP(hipStreamSynchronize(N.s));
     })
 }
@@ -371,13 +370,12 @@ int rt_net_gradient(rt_net* n, const int* dims, const float* x, const float* tar
         Net& N = N_(n);
         shape(N, dims);
         const size_t P = P_of(dims);
-        DBuf xin;
-        xin.alloc(sizeof(float) * P * 4);
+        N.xin.ensure(sizeof(float) * P * 4);
         N.T.ensure(sizeof(float) * P * 3);
-        RT_HIP(hipMemcpyAsync(xin.p, x, sizeof(float) * P * 4, hipMemcpyHostToDevice, N.s));
+        RT_HIP(hipMemcpyAsync(N.xin.p, x, sizeof(float) * P * 4, hipMemcpyHostToDevice, N.s));
         RT_HIP(hipMemcpyAsync(N.T.p, target, sizeof(float) * P * 3, hipMemcpyHostToDevice, N.s));
         RT_HIP(hipMemsetAsync(N.G.p, 0, sizeof(float) * N.nparam, N.s));
-        launch_pack_input(P, xin.as<float>(), mb(N.F), N.s);
+        launch_pack_input(P, N.xin.as<float>(), mb(N.F), N.s);
         forward(N, N.s);
         *loss = loss_grad(N, N.T.as<float>(), 1.f, N.s);
         backward(N, N.s);
