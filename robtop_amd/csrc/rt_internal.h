@@ -282,6 +282,10 @@ void launch_sensitivity(const Geom& g, Vec3<const T> U, const float* rho, const 
 void launch_filter(const Geom& g, const float* gin, const uint8_t* eflag, float R, float* gout, hipStream_t s);
 void launch_oc_trial(const Geom& g, const float* rho, const float* sens, const uint8_t* eflag, float thr, float step,
                      float damp, float rhomin, float* rho_out, double* partials, int nparts, hipStream_t s);
+constexpr int kOcTrials = 7;        // three steps of a bisection
+void launch_oc_volumes(const Geom& g, const float* rho, const float* sens, const uint8_t* eflag, float gmax,
+                       const float* thr, float step, float damp, float rhomin, double* partials, int nparts,
+                       hipStream_t s);
 void launch_maxabs(const Geom& g, const float* a, const uint8_t* eflag, double* partials, int nparts, hipStream_t s);
 void launch_sum_active(const Geom& g, const float* a, const uint8_t* eflag, double* partials, int nparts,
                        hipStream_t s);
