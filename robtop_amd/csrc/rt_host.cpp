@@ -128,6 +128,10 @@ struct Hier {
     // direction), projected force and the previous step's force, all [3][nload]
     DBuf load_slots, load_nrm, pm_fs, pm_old;
     DBuf ocpart;                     // density update: partial sums of a pass's trials
+    // scalars of the CG on the device, kBatchMax of each: r.z, p.Ap, r.r, alpha, beta. The step lengths and
+    // directions are computed there, so an iteration waits for the device once (for r.r) instead of three times
+    DBuf cgs;
+    double* cg(int k) const { return cgs.as<double>() + k * kBatchMax; }
     DBuf gram;                       // block Lanczos: partial sums of the projections
     // no-support modes: the admissible rigid motions of the load nodes
     // (compact [k][c * nload + i], nrd of them) and the finest nodes' rigid
@@ -795,19 +799,24 @@ static double sum_partials_host(Hier& H, int np) {
     return v;
 }
 
-// r . z after precondition<float>(H, pc, pre, post): from the last fine
-// sweep's partials when it wrote them, else a separate pass over both vectors
-static double precond_rz(Hier& H, LevelVecs<float>& pc, int post, size_t n) {
-    if (!rz_fused(H, post)) {
-        launch_dot_partials_t<float, float>(pc.F.data(), pc.U.data(), n, H.partials.as<double>(), kStreamBlocks, H.s,
-                                            vec_chunks(H));
-        return sum_partials_host(H, kStreamBlocks);
-    }
-    launch_sum_partials(H.rzpart.as<double>(), H.rzpart_n, H.scal.as<double>(), H.s);
-    double v;
-    RT_HIP(hipMemcpyAsync(&v, H.scal.p, sizeof(double), hipMemcpyDeviceToHost, H.s));
+enum CgScalar { kCgRz = 0, kCgPq, kCgRr, kCgAlpha, kCgBeta, kCgScalars };
+using CgValues = double[kCgScalars][kBatchMax];
+static void cg_read(Hier& H, CgValues& v) {
+    RT_HIP(hipMemcpyAsync(v, H.cgs.p, sizeof(v), hipMemcpyDeviceToHost, H.s));
     RT_HIP(hipStreamSynchronize(H.s));
-    return v;
+}
+
+// partial sums of r . z after precondition<float>(H, pc, pre, post): the last fine
+// sweep's when it wrote them, else of a separate pass over both vectors
+static const double* precond_rz_parts(Hier& H, LevelVecs<float>& pc, int post, size_t n, int* np) {
+    if (rz_fused(H, post)) {
+        *np = H.rzpart_n;
+        return H.rzpart.as<double>();
+    }
+    launch_dot_partials_t<float, float>(pc.F.data(), pc.U.data(), n, H.partials.as<double>(), kStreamBlocks, H.s,
+                                        vec_chunks(H));
+    *np = kStreamBlocks;
+    return H.partials.as<double>();
 }
 
 // ---------------------------------------------------------------------------
@@ -1083,12 +1092,16 @@ template <> struct KV<float> {
 };
 
 template <typename TV>
-static double apply_dot(Hier& H, V3<TV>& X, V3<TV>& Y) {
+static int apply_partials(Hier& H, V3<TV>& X, V3<TV>& Y) {
     Level& L0 = H.lv[0];
     int np = 0;
     launch_fine_apply_modal<TV>(L0.g, X.cv(), Y.v(), H.rhop.as<float>(), L0.vflag.as<uint8_t>(), H.partials.as<double>(), &np,
                           H.s);
-    return sum_partials_host(H, np);
+    return np;
+}
+template <typename TV>
+static double apply_dot(Hier& H, V3<TV>& X, V3<TV>& Y) {
+    return sum_partials_host(H, apply_partials<TV>(H, X, Y));
 }
 
 static double true_rel_residual(Hier& H) {
@@ -1398,19 +1411,28 @@ static void pcg_reliable(Hier& H, double tol, int maxit, int pre, int post, rt_s
         H.cg_beta.clear();
         launch_fill<float>(H.dx32.data(), 0.f, n, H.s);
         precondition<float>(H, pc, pre, post);
-        double rz = precond_rz(H, pc, post, n);
+        H.cgs.ensure(sizeof(CgValues));
+        int npz = 0;
+        const double* zp = precond_rz_parts(H, pc, post, n, &npz);
+        launch_sum_partials(zp, npz, H.cg(kCgRz), H.s);
         launch_convert<float, float>(pc.U.data(), H.p32.data(), n, H.s);
         bool flushed = false;
         double apend = 0.0;
         for (it = 1; it <= maxit; it++) {
-            const double pq = apply_dot<float>(H, H.p32, H.q32);
-            if (!(pq > 0)) throw std::domain_error("PCG breakdown: p.Ap <= 0");
-            const double alpha = rz / pq;
-            H.cg_alpha.push_back(alpha);
-            launch_pcg_ru_r(pc.F.data(), H.q32.data(), alpha, n, H.partials.as<double>(), ns, H.s, vec_chunks(H));
-            apend = alpha;
+            const bool on = true;
+            const int npq = apply_partials<float>(H, H.p32, H.q32);
+            launch_sum_ratio(H.partials.as<double>(), npq, H.cg(kCgPq), H.cg(kCgRz), H.cg(kCgAlpha), false, H.s);
+            launch_pcg_ru_r(pc.F.data(), H.q32.data(), Coefs(H.cg(kCgAlpha), &on, 1), n, H.partials.as<double>(), ns,
+                            H.s, vec_chunks(H));
+            launch_sum_partials(H.partials.as<double>(), ns, H.cg(kCgRr), H.s);
+            CgValues v;
+            cg_read(H, v);
+            if (!(v[kCgPq][0] > 0)) throw std::domain_error("PCG breakdown: p.Ap <= 0");
+            if (it > 1) H.cg_beta.push_back(v[kCgBeta][0]);
+            apend = v[kCgAlpha][0];
+            H.cg_alpha.push_back(apend);
             flushed = false;
-            const double rn = std::sqrt(sum_partials_host(H, ns));
+            const double rn = std::sqrt(v[kCgRr][0]);
             rel = rn / nb;
             if (rel <= tol || rn < RT_REPLACE_DROP * rmax) {
                 launch_pcg_flush_x(H.x64.data(), H.dx32.data(), n, H.s, H.p32.data(), apend);
@@ -1426,11 +1448,11 @@ static void pcg_reliable(Hier& H, double tol, int maxit, int pre, int post, rt_s
             }
             if (it == maxit) break;
             precondition<float>(H, pc, pre, post);
-            const double rz_new = precond_rz(H, pc, post, n);
-            const double beta = rz_new / rz;
-            H.cg_beta.push_back(beta);
-            rz = rz_new;
-            launch_pcg_p_dx(H.p32.data(), pc.U.data(), beta, H.dx32.data(), apend, n, H.s, vec_chunks(H));
+            zp = precond_rz_parts(H, pc, post, n, &npz);
+            // (r.r's place takes r.z as well: the sum itself is not needed)
+            launch_sum_ratio(zp, npz, H.cg(kCgRr), H.cg(kCgRz), H.cg(kCgBeta), true, H.s);
+            launch_pcg_p_dx(H.p32.data(), pc.U.data(), Coefs(H.cg(kCgBeta), &on, 1), H.dx32.data(), apend, n, H.s,
+                            vec_chunks(H));
             apend = 0.0;
         }
         if (!flushed) launch_pcg_flush_x(H.x64.data(), H.dx32.data(), n, H.s, H.p32.data(), apend);
@@ -2868,7 +2890,8 @@ static void pcg_batch(Hier& H, int nb, double tol, int maxit, int pre, int post,
     Level& L0 = H.lv[0];
     const size_t n = (size_t)3 * L0.g.N;
     const int np = 1024, npa = batch_part_stride(H);
-    double nf[kBatchMax], rr[kBatchMax], rz[kBatchMax], pq[kBatchMax], c[kBatchMax] = {};
+    double nf[kBatchMax], rr[kBatchMax];
+    H.cgs.ensure(sizeof(CgValues));
     double* part = H.bpart.as<double>();
     bool act[kBatchMax];
     launch_fill<double>(H.bx.data(), 0.0, n * nb, H.s);
@@ -2887,7 +2910,7 @@ static void pcg_batch(Hier& H, int nb, double tol, int maxit, int pre, int post,
         precondition_batch(H, nb, pre, post);
         launch_dot_partials_t<double, float>(H.br.data(), L0.bU.data(), n, part, np, H.s, nullptr, nb, npa);
         launch_convert<float, double>(L0.bU.data(), H.bp.data(), n * nb, H.s);
-        batch_sums(H, nb, np, npa, rz);
+        launch_sum_partials(part, np, H.cg(kCgRz), H.s, nb, npa);
     }
     for (int it = 1; it <= maxit && live; it++) {
         int npq = 0;
@@ -2895,22 +2918,21 @@ static void pcg_batch(Hier& H, int nb, double tol, int maxit, int pre, int post,
             launch_fine_apply_modal<double>(L0.g, H.bp.cv(b), H.bq.v(b), H.rhop.as<float>(), L0.vflag.as<uint8_t>(),
                                             part + (size_t)b * npa, &npq, H.s, k, npa);
         });
-        batch_sums(H, nb, npq, npa, pq);
-        for (int b = 0; b < nb; b++) {
-            if (!act[b]) continue;
-            if (!(pq[b] > 0)) throw std::domain_error("PCG breakdown: p.Ap <= 0");
-            c[b] = rz[b] / pq[b];
-        }
+        launch_sum_ratio(part, npq, H.cg(kCgPq), H.cg(kCgRz), H.cg(kCgAlpha), false, H.s, nb, npa);
         active_runs(act, nb, [&](int b, int k) {
-            launch_pcg_update_x_r<double, float>(H.bx.at(b), H.br.at(b), H.bp.at(b), H.bq.at(b), Coefs(c + b, k), n,
-                                                 part + (size_t)b * npa, np, L0.bF.at(b), H.s, k, npa);
+            launch_pcg_update_x_r<double, float>(H.bx.at(b), H.br.at(b), H.bp.at(b), H.bq.at(b),
+                                                 Coefs(H.cg(kCgAlpha) + b, act + b, k), n, part + (size_t)b * npa, np,
+                                                 L0.bF.at(b), H.s, k, npa);
         });
-        batch_sums(H, nb, np, npa, rr);
+        launch_sum_partials(part, np, H.cg(kCgRr), H.s, nb, npa);
+        CgValues v;
+        cg_read(H, v);
         live = 0;
         for (int b = 0; b < nb; b++) {
             if (!act[b]) continue;
+            if (!(v[kCgPq][b] > 0)) throw std::domain_error("PCG breakdown: p.Ap <= 0");
             iters[b] = it;
-            if (std::sqrt(rr[b]) <= tol * nf[b]) act[b] = false;
+            if (std::sqrt(v[kCgRr][b]) <= tol * nf[b]) act[b] = false;
             else live++;
         }
         if (!live) break;
@@ -2919,15 +2941,10 @@ static void pcg_batch(Hier& H, int nb, double tol, int maxit, int pre, int post,
             launch_dot_partials_t<double, float>(H.br.at(b), L0.bU.at(b), n, part + (size_t)b * npa, np, H.s, nullptr, k,
                                                  npa);
         });
-        double rzn[kBatchMax];
-        batch_sums(H, nb, np, npa, rzn);
-        for (int b = 0; b < nb; b++) {
-            if (!act[b]) continue;
-            c[b] = rzn[b] / rz[b];
-            rz[b] = rzn[b];
-        }
+        launch_sum_ratio(part, np, H.cg(kCgRr), H.cg(kCgRz), H.cg(kCgBeta), true, H.s, nb, npa);
         active_runs(act, nb, [&](int b, int k) {
-            launch_pcg_update_p<double, float>(H.bp.at(b), L0.bU.at(b), Coefs(c + b, k), n, H.s, k);
+            launch_pcg_update_p<double, float>(H.bp.at(b), L0.bU.at(b), Coefs(H.cg(kCgBeta) + b, act + b, k), n, H.s,
+                                               k);
         });
     }
     // true residuals |f_b - K x_b| / |f_b|
@@ -2954,12 +2971,12 @@ static void pcg_batch_reliable(Hier& H, int nb, double tol, int maxit, int pre, 
     const size_t n = (size_t)3 * L0.g.N;
     const int np = 1024, ns = kStreamBlocks, npa = batch_part_stride(H);
     double* part = H.bpart.as<double>();
-    double nf[kBatchMax], rmax[kBatchMax], best[kBatchMax], rz[kBatchMax], pq[kBatchMax], rn[kBatchMax],
-        rt[kBatchMax];
+    double nf[kBatchMax], rmax[kBatchMax], best[kBatchMax], rt[kBatchMax];
+    H.cgs.ensure(sizeof(CgValues));
     bool act[kBatchMax], bad[kBatchMax], dirty[kBatchMax];
     // apend[b]: the step whose alpha p is not yet on dx (added by the next
     // direction update or by the flush, as in pcg_reliable)
-    double apend[kBatchMax] = {}, c[kBatchMax] = {};
+    double apend[kBatchMax] = {};
     launch_fill<double>(H.bx.data(), 0.0, n * nb, H.s);
     launch_fill<float>(H.bdx32.data(), 0.f, n * nb, H.s);
     launch_convert<double, float>(H.bb.data(), L0.bF.data(), n * nb, H.s);
@@ -2998,7 +3015,7 @@ static void pcg_batch_reliable(Hier& H, int nb, double tol, int maxit, int pre, 
         precondition_batch(H, nb, pre, post);
         launch_dot_partials_t<float, float>(L0.bF.data(), L0.bU.data(), n, part, ns, H.s, vec_chunks(H), nb, npa);
         launch_convert<float, float>(L0.bU.data(), H.bp32.data(), n * nb, H.s);
-        batch_sums(H, nb, ns, npa, rz);
+        launch_sum_partials(part, ns, H.cg(kCgRz), H.s, nb, npa);
     }
     for (int it = 1; it <= maxit && live; it++) {
         int npq = 0;
@@ -3006,18 +3023,21 @@ static void pcg_batch_reliable(Hier& H, int nb, double tol, int maxit, int pre, 
             launch_fine_apply_modal<float>(L0.g, H.bp32.cv(b), H.bq32.v(b), H.rhop.as<float>(),
                                            L0.vflag.as<uint8_t>(), part + (size_t)b * npa, &npq, H.s, k, npa);
         });
-        batch_sums(H, nb, npq, npa, pq);
+        launch_sum_ratio(part, npq, H.cg(kCgPq), H.cg(kCgRz), H.cg(kCgAlpha), false, H.s, nb, npa);
+        active_runs(act, nb, [&](int b, int k) {
+            launch_pcg_ru_r(L0.bF.at(b), H.bq32.at(b), Coefs(H.cg(kCgAlpha) + b, act + b, k), n,
+                            part + (size_t)b * npa, ns, H.s, vec_chunks(H), k, npa);
+        });
+        launch_sum_partials(part, ns, H.cg(kCgRr), H.s, nb, npa);
+        CgValues v;
+        cg_read(H, v);
+        double* rn = v[kCgRr];
         for (int b = 0; b < nb; b++) {
             if (!act[b]) continue;
-            if (!(pq[b] > 0)) throw std::domain_error("PCG breakdown: p.Ap <= 0");
-            apend[b] = rz[b] / pq[b];
+            if (!(v[kCgPq][b] > 0)) throw std::domain_error("PCG breakdown: p.Ap <= 0");
+            apend[b] = v[kCgAlpha][b];
             dirty[b] = true;
         }
-        active_runs(act, nb, [&](int b, int k) {
-            launch_pcg_ru_r(L0.bF.at(b), H.bq32.at(b), Coefs(apend + b, k), n, part + (size_t)b * npa, ns, H.s,
-                            vec_chunks(H), k, npa);
-        });
-        batch_sums(H, nb, ns, npa, rn);
         bool rep[kBatchMax] = {};
         int nrep = 0;
         for (int b = 0; b < nb; b++) {
@@ -3052,19 +3072,13 @@ static void pcg_batch_reliable(Hier& H, int nb, double tol, int maxit, int pre, 
             launch_dot_partials_t<float, float>(L0.bF.at(b), L0.bU.at(b), n, part + (size_t)b * npa, ns, H.s,
                                                 vec_chunks(H), k, npa);
         });
-        double rzn[kBatchMax];
-        batch_sums(H, nb, ns, npa, rzn);
-        for (int b = 0; b < nb; b++)
-            if (act[b]) c[b] = rzn[b] / rz[b];
+        launch_sum_ratio(part, ns, H.cg(kCgRr), H.cg(kCgRz), H.cg(kCgBeta), true, H.s, nb, npa);
         active_runs(act, nb, [&](int b, int k) {
-            launch_pcg_p_dx(H.bp32.at(b), L0.bU.at(b), Coefs(c + b, k), H.bdx32.at(b), Coefs(apend + b, k), n, H.s,
-                            vec_chunks(H), k);
+            launch_pcg_p_dx(H.bp32.at(b), L0.bU.at(b), Coefs(H.cg(kCgBeta) + b, act + b, k), H.bdx32.at(b),
+                            Coefs(apend + b, k), n, H.s, vec_chunks(H), k);
         });
-        for (int b = 0; b < nb; b++) {
-            if (!act[b]) continue;
-            apend[b] = 0.0;
-            rz[b] = rzn[b];
-        }
+        for (int b = 0; b < nb; b++)
+            if (act[b]) apend[b] = 0.0;
     }
     for (int b = 0; b < nb; b++)
         if (dirty[b]) launch_pcg_flush_x(H.bx.at(b), H.bdx32.at(b), n, H.s, H.bp32.at(b), apend[b]);
@@ -3425,7 +3439,7 @@ int rt_update_densities(rt_hier* h, float vgoal, float step, float damp, float r
         // half at 2k + 1. An exponent above one could overflow the factor of a
         // small multiplier (down to 2^-31 of the largest sensitivity), so those, and
         // sensitivities without a finite positive maximum, go one trial at a time.
-        // About ten passes instead of 28 and as many waits for the device: 0.9 -> 0.5 ms
+        // About ten passes instead of 28 and as many waits for the device: 0.48 -> 0.22 ms
         // an update at 64 x 32 x 32 elements, 6.3 -> 2.4 ms at 511 x 256 x 256.
         if (gmax > 0.f && gmax <= std::numeric_limits<float>::max() && 1.f / gmax <= std::numeric_limits<float>::max() &&
             damp > 0.f && damp <= 1.f) {

@@ -221,14 +221,23 @@ void launch_dot_partials(const double* a, const double* b, size_t n, double* par
 constexpr int kBatchMax = 8;
 struct Coefs {
     double v[kBatchMax];
+    const double* dev = nullptr;
     Coefs() = default;
     Coefs(double x) : v{x} {}
     explicit Coefs(const double* x, int n) : v{} { for (int i = 0; i < n; i++) v[i] = x[i]; }
+    // n coefficients in device memory (written by launch_sum_ratio): read where on[i], 0 elsewhere
+    Coefs(const double* d, const bool* on, int n) : v{}, dev(d) { for (int i = 0; i < n; i++) v[i] = on[i]; }
+    __device__ double at(unsigned b) const { return dev && v[b] != 0 ? dev[b] : v[b]; }
 };
 template <typename TA, typename TB>
 void launch_dot_partials_t(const TA* a, const TB* b, size_t n, double* partials, int nparts, hipStream_t s,
                            const uint8_t* chunk = nullptr, int nb = 1, int pstride = 0);
 void launch_sum_partials(const double* partials, int nparts, double* out, hipStream_t s, int nb = 1, int pstride = 0);
+// the same sums with a step's coefficient of the CG from them, on the device: out =
+// sum and, for a step length (direction = false), coef = rz / sum; for a new
+// direction, coef = sum / rz and rz = sum
+void launch_sum_ratio(const double* partials, int nparts, double* out, double* rz, double* coef, bool direction,
+                      hipStream_t s, int nb = 1, int pstride = 0);
 template <typename T, typename TZ>
 void launch_pcg_update_x_r(T* x, T* r, const T* p, const T* q, Coefs alpha, size_t n, double* partials, int nparts,
                            TZ* rz_out, hipStream_t s, int nb = 1, int pstride = 0);
