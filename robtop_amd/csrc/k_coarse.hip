@@ -813,8 +813,9 @@ __global__ void k_gather_rows(const int* __restrict__ rowslot, int nrows, Vec3<c
 
 // U = Ainv f at the coarsest nodes, a workgroup per row. Bound by the matrix,
 // read from the last-level cache; a wave per row walked 50 to 65 loads a lane with
-// a few in flight. 3,264 unknowns: 25.9 us with a wave per row, 21.9 us so; 4,131:
-// 41.2 and 32.5 us (4.2 TB/s).
+// a few in flight. 4,131 unknowns (136 MB) below 64 x 32 x 32 elements: 25.9 us with
+// a wave per row, 21.9 us so; below 256 x 128 x 128, whose vectors displace the matrix
+// between cycles: 41.2 and 32.5 us (4.2 TB/s).
 template <typename T>
 __global__ void __launch_bounds__(256) k_dense_gemv(const double* __restrict__ A, int n, int ld,
                                                     const double* __restrict__ f, const int* __restrict__ rowslot,
@@ -1548,8 +1549,8 @@ __global__ void k_gather_rows_b(const int* __restrict__ rowslot, int nrows, cons
 
 // Four rows a workgroup: the vectors, not the matrix, bound the batch (each row
 // reads all of them from L2), so four rows share each load of a vector. Eight
-// vectors of 4,131 unknowns: 116 us with a row a wave, 39 us so; five of 1,500: 39 and
-// 14 us.
+// vectors below a torus of 128 elements a side: 116 us with a row a wave, 39 us so;
+// five below 90 x 41 x 37 elements: 39 and 14 us.
 // The sums of a vector do not depend on NB.
 constexpr int kGemvRows = 4;
 template <typename T, int NB>
