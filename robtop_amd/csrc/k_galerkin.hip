@@ -119,46 +119,77 @@ void launch_galerkin4_fix(const Geom& gf, const int ec[3], const float* rhop, co
     RT_HIP(hipGetLastError());
 }
 
-// x2 Galerkin on element matrices: one block per parent element, the 8 child
-// matrices staged in LDS, one thread per output entry.
-__global__ void __launch_bounds__(576) k_galerkin2(const double* __restrict__ KEf, int efx, int efy, int efz,
-                                                   double* __restrict__ KEp, int epx, int epy, int epz) {
-    const int e = blockIdx.x;
-    const int nEp = epx * epy * epz, nEf = efx * efy * efz;
-    const int x = e % epx, y = (e / epx) % epy, z = e / (epx * epy);
-    const int t = threadIdx.x;
-    __shared__ double Kc[8][576];
-    for (int c = 0; c < 8; c++) {
-        const int cx = 2 * x + (c & 1), cy = 2 * y + ((c >> 1) & 1), cz = 2 * z + (c >> 2);
-        double v = 0;
-        if (cx < efx && cy < efy && cz < efz) v = KEf[(size_t)t * nEf + cx + efx * (cy + efy * cz)];
-        Kc[c][t] = v;
-    }
-    __syncthreads();
-    const int A = t / 72, ra = (t / 24) % 3, B = (t % 24) / 3, sb = t % 3;
-    double acc = 0;
+// x2 Galerkin on element matrices. Output entry (3A + ra, 3B + sb) of a parent
+// takes the entries (3i + ra, 3j + sb) of its eight children, so a workgroup takes
+// one (ra, sb) for 16 parents of a row: the 64 entries (i, j) of their 32 x 2 x 2
+// children are staged in LDS in runs of 32 values (the matrices lie entry by entry,
+// elements contiguous), each matrix entry read once. A thread computes half the
+// columns B of a row A of one parent; a wave's four rows A read the same LDS
+// values. Bound by the read of the child matrices. One parent a workgroup read two
+// neighbouring values at a time: the four levels below 511 x 256 x 256 elements took
+// 6.0 ms, 1.8 ms so (the first, 128 x 64 x 64 children, 1.6 ms: 1.7 TB/s).
+constexpr int kG2Run = 16;
+template <int HB>
+__device__ __forceinline__ void galerkin2_cols(const double (&K)[64][8][kG2Run], int A, int p, double (&acc)[4]) {
+#pragma unroll
     for (int c = 0; c < 8; c++) {
         const int ox = c & 1, oy = (c >> 1) & 1, oz = c >> 2;
+#pragma unroll 2
         for (int i = 0; i < 8; i++) {
             const int pix = ox + (i & 1), piy = oy + ((i >> 1) & 1), piz = oz + (i >> 2);
             const int wi = ((A & 1) ? pix : 2 - pix) * ((A & 2) ? piy : 2 - piy) * ((A & 4) ? piz : 2 - piz);
-            if (wi == 0) continue;
-            double s = 0;
+            double s[4] = {0, 0, 0, 0};
+#pragma unroll
             for (int j = 0; j < 8; j++) {
                 const int pjx = ox + (j & 1), pjy = oy + ((j >> 1) & 1), pjz = oz + (j >> 2);
-                const int wj = ((B & 1) ? pjx : 2 - pjx) * ((B & 2) ? pjy : 2 - pjy) * ((B & 4) ? pjz : 2 - pjz);
-                if (wj == 0) continue;
-                s += Kc[c][(3 * i + ra) * 24 + 3 * j + sb] * (double)wj;
+                if ((HB ? pjz : 2 - pjz) == 0) continue;
+                const double k = K[8 * i + j][c][p];
+#pragma unroll
+                for (int b = 0; b < 4; b++) {
+                    const int wj = ((b & 1) ? pjx : 2 - pjx) * ((b & 2) ? pjy : 2 - pjy) * (HB ? pjz : 2 - pjz);
+                    if (wj) s[b] += k * (double)wj;
+                }
             }
-            acc += s * (double)wi;
+#pragma unroll
+            for (int b = 0; b < 4; b++) acc[b] += s[b] * (double)wi;
         }
     }
-    KEp[(size_t)t * nEp + e] = acc * (1.0 / 64.0);
+}
+__global__ void __launch_bounds__(256) k_galerkin2(const double* __restrict__ KEf, int efx, int efy, int efz,
+                                                   double* __restrict__ KEp, int epx, int epy, int epz) {
+    __shared__ double K[64][8][kG2Run];
+    const int runs = (epx + kG2Run - 1) / kG2Run, row = blockIdx.x / runs;
+    const int x0 = (blockIdx.x % runs) * kG2Run, y = row % epy, z = row / epy;
+    const int ra = blockIdx.y / 3, sb = blockIdx.y % 3;
+    const size_t nEp = (size_t)epx * epy * epz, nEf = (size_t)efx * efy * efz;
+    const int t = threadIdx.x;
+    {
+        const int cx = 2 * x0 + (t & 31);
+#pragma unroll 8
+        for (int k = t >> 5; k < 256; k += 8) {
+            const int ij = k >> 2, cy = 2 * y + (k & 1), cz = 2 * z + ((k >> 1) & 1);
+            double v = 0;
+            if (cx < efx && cy < efy && cz < efz)
+                v = KEf[(size_t)((3 * (ij >> 3) + ra) * 24 + 3 * (ij & 7) + sb) * nEf + cx +
+                        (size_t)efx * (cy + (size_t)efy * cz)];
+            K[ij][(t & 1) + 2 * (k & 3)][(t & 31) >> 1] = v;
+        }
+    }
+    __syncthreads();
+    const int p = t & 15, A = (t >> 4) & 7, hb = t >> 7;
+    double acc[4] = {0, 0, 0, 0};
+    if (hb) galerkin2_cols<1>(K, A, p, acc);
+    else galerkin2_cols<0>(K, A, p, acc);
+    if (x0 + p >= epx) return;
+    const size_t e = x0 + p + (size_t)epx * (y + (size_t)epy * z);
+#pragma unroll
+    for (int b = 0; b < 4; b++)
+        KEp[(size_t)((3 * A + ra) * 24 + 3 * (4 * hb + b) + sb) * nEp + e] = acc[b] * (1.0 / 64.0);
 }
 
 void launch_galerkin2(const double* KEf, const int ef[3], double* KEp, const int ep[3], hipStream_t s) {
-    int nEp = ep[0] * ep[1] * ep[2];
-    hipLaunchKernelGGL(k_galerkin2, dim3(nEp), dim3(576), 0, s, KEf, ef[0], ef[1], ef[2], KEp, ep[0], ep[1], ep[2]);
+    hipLaunchKernelGGL(k_galerkin2, dim3((ep[0] + kG2Run - 1) / kG2Run * ep[1] * ep[2], 9), dim3(256), 0, s, KEf,
+                       ef[0], ef[1], ef[2], KEp, ep[0], ep[1], ep[2]);
     RT_HIP(hipGetLastError());
 }
 
