@@ -1875,10 +1875,8 @@ int rt_set_density_box(rt_hier* h, const float* rho_box) {
     RT_TRY({
         need(rho_box);
         Hier& H = H_(h);
-        std::vector<float> box(rho_box, rho_box + H.lv[0].ne_box());
-        for (size_t e = 0; e < box.size(); e++) if (!H.lv[0].eact[e]) box[e] = 0.f;
-        upload_box<float>(H, H.lv[0].g, 1, box.data(), H.rho.as<float>());
-        launch_rhop(H.lv[0].g, H.rho.as<float>(), H.eflag.as<uint8_t>(), H.p, H.rhop.as<float>(), H.s);
+        upload_box<float>(H, H.lv[0].g, 1, rho_box, H.rho.as<float>());
+        launch_mask_rhop(H.lv[0].g, H.rho.as<float>(), H.eflag.as<uint8_t>(), H.p, H.rhop.as<float>(), H.s);
         RT_HIP(hipStreamSynchronize(H.s));
         H.stencil_ready = false;
     })

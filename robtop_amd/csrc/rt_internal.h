@@ -285,6 +285,7 @@ void launch_assemble(const Geom& g, const double* KEc, const int e[3], const uin
 // k_simp.hip
 void set_ke_simp(const double* ke576, hipStream_t s);
 void launch_rhop(const Geom& g, const float* rho, const uint8_t* eflag, float p, float* rhop, hipStream_t s);
+void launch_mask_rhop(const Geom& g, float* rho, const uint8_t* eflag, float p, float* rhop, hipStream_t s);
 template <typename T>
 void launch_sensitivity(const Geom& g, Vec3<const T> U, const float* rho, const uint8_t* eflag, float p, float* sens,
                         hipStream_t s);
