@@ -239,7 +239,7 @@ def pmc_summary(fetch_csv, write_csv, size):
     fa, fc = per_kernel(fetch_csv, "FETCH_SIZE")
     wa, wc = per_kernel(write_csv, "WRITE_SIZE")
     kf, kw = fc / CALIB_BYTES, wc / CALIB_BYTES
-    kname = "k_fine_gs_tile" if any("k_fine_gs_tile" in k for k in fa) else "k_fine_gs_pair"
+    kname = next(n for n in ("k_fine_gs_tile", "k_fine_gs_row", "k_fine_gs_pair") if any(n in k for k in fa))
     launches = 2 if kname == "k_fine_gs_tile" else 4
     gs = [k for k in fa if kname in k]
     fetch = sum(sum(fa[k]) for k in gs) / sum(len(fa[k]) for k in gs) / kf
@@ -475,7 +475,7 @@ def main():
     # (one z-parity class each, half the nodes), the colour-pair smoother as four
     # (one (y, z) parity class each); each launch is charged its share.
     n_launch = 2 if a.fine_smoother == "tiled" else 4
-    kname = "k_fine_gs_tile" if a.fine_smoother == "tiled" else "k_fine_gs_pair"
+    kname = "k_fine_gs_tile" if a.fine_smoother == "tiled" else "k_fine_gs_row"
     sweep_bytes = levels[0]["nodes"] * (9 * 4 + 1) + 4 * levels[0]["elements"]
     launch_bytes = sweep_bytes / n_launch
     launch_ms = t_sweep / n_launch
