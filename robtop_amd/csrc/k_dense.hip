@@ -63,6 +63,8 @@ __device__ __forceinline__ double gj_rcp(double x) {
 // pivot columns, which their 16 threads put into LDS. 4 x 4 blocks, since the
 // LDS reads of the pivot columns are what a step takes: 8 values a thread and
 // column against 17 with a thread per row.
+// The pivot block is scaled by a power of two (exact) so that its determinant is
+// in range for every stiffness whose inverse is.
 __device__ __forceinline__ void gj_invert(const double (*S)[GB + 1], double (*col)[2][GB], double* __restrict__ D,
                                           int* __restrict__ info) {
     const int ti = threadIdx.x >> 4, tj = threadIdx.x & 15;
@@ -82,7 +84,10 @@ __device__ __forceinline__ void gj_invert(const double (*S)[GB + 1], double (*co
                 for (int i = 0; i < 4; i++) { c[0][4 * ti + i] = a[i][2 * h]; c[1][4 * ti + i] = a[i][2 * h + 1]; }
             }
             __syncthreads();
-            const double d00 = c[0][p], d01 = c[1][p], d11 = c[1][p + 1];
+            const double t00 = c[0][p];
+            const int sx = -__builtin_amdgcn_frexp_exp(t00);
+            const double d00 = __builtin_ldexp(t00, sx), d01 = __builtin_ldexp(c[1][p], sx),
+                         d11 = __builtin_ldexp(c[1][p + 1], sx);
             double r0[4], r1[4], k0[4], k1[4];
 #pragma unroll
             for (int i = 0; i < 4; i++) {
@@ -91,7 +96,7 @@ __device__ __forceinline__ void gj_invert(const double (*S)[GB + 1], double (*co
             }
             const double det = d00 * d11 - d01 * d01;
             bad = bad || !(d00 > 0) || !(det > 0);
-            const double rd = gj_rcp(det), e00 = d11 * rd, e01 = -d01 * rd, e11 = d00 * rd;
+            const double rd = __builtin_ldexp(gj_rcp(det), sx), e00 = d11 * rd, e01 = -d01 * rd, e11 = d00 * rd;
             double x0[4], x1[4];
 #pragma unroll
             for (int i = 0; i < 4; i++) {                                // W

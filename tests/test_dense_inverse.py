@@ -90,3 +90,40 @@ def test_zero_stiffness_is_refused():
     with pytest.raises(rt.RobtopError, match="not positive definite"):
         hg.update_stencil()
     hg.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("exponent", [-540, -530, 0, 520])
+def test_stiffness_far_from_one(exponent):
+    """Young's moduli whose pivots' products pass double precision's range, where the pivots and their reciprocals
+    do not: FP64 V-cycles against the oracle's, to the 1e-10 of the other FP64 comparisons."""
+    import oracle
+    import robtop_amd as rt
+    print(f"[dense] Young's modulus 2^{exponent}", flush=True)
+    a = solid(64, 20, 56, 24, True)
+    bits = cube_bits(a)
+    o, g = oracle.Hierarchy(64, bits), rt.HierarchyGrid.genFromMesh(bits, 64)
+    nx, ny, nz = g[0].nodes
+    eact, vact = g[0].masks()
+    fixed = np.zeros((nz, ny, nx), bool)
+    fixed[:, :, 0] = True
+    fixed = fixed.reshape(-1) & vact
+    rng = np.random.default_rng(5)
+    rho = (rng.uniform(0.2, 1.0, eact.size) * eact).astype(np.float32)
+    f = rng.standard_normal((3, vact.size)) * (vact & ~fixed)
+    for h in (o, g):
+        h.set_material(2.0 ** exponent, 0.4, 3.0)
+    o.set_fixed(fixed); g.set_support(fixed)
+    o.set_rho(rho); g.set_density(rho)
+    o.set_rhop(g.get_rhop())
+    zero = np.zeros_like(f)
+    o.set_vec(0, 1, f); g.set_force(f)
+    o.set_vec(0, 0, zero); g.set_displacement(zero)
+    g.set_precision(64)
+    g.update_stencil(); o.update_stencil()
+    for _ in range(2):
+        rg, ro = g.v_cycle(1, 1), o.v_cycle(1, 1)
+        assert np.isfinite(ro) and abs(rg - ro) <= 1e-10 * ro, (rg, ro)
+    u, ref = g.get_displacement(), o.get_vec(0, 0)
+    assert np.abs(u - ref).max() <= 1e-10 * np.abs(ref).max()
+    g.close()
