@@ -362,11 +362,13 @@ __global__ void __launch_bounds__(256) k_conv_wgrad(Dims D, const uint16_t* __re
 #pragma unroll
             for (int nb = 0; nb < NB; nb++) a[nb][j] = in ? (short)G[pk * COUT + nb * 16 + m] : (short)0;
         }
-        // X at xk + dx0 .. xk + dx0 + TX + 2: tap q uses entries q .. q + 3
+        // X at xk + dx0 .. xk + dx0 + TX + 2: tap q uses entries q .. q + 3. The value
+        // of the row's last position is no term of a tap at dx = -1: its G lies past
+        // the row, and 0 times an infinity is not 0.
 #pragma unroll
         for (int j = 0; j < TX + 3; j++) {
             const int xn = xk + dx0 + j;
-            const bool ok = rowok && xn >= 0 && xn < nx;
+            const bool ok = rowok && xn >= 0 && xn < nx && (TX > 1 || xk + j < nx);
             const size_t pn = ok ? nrow + xn : 0;
 #pragma unroll
             for (int kb = 0; kb < KB; kb++) b[kb][j] = ok ? (short)X[pn * CIN + kb * 16 + m] : (short)0;
@@ -377,7 +379,11 @@ __global__ void __launch_bounds__(256) k_conv_wgrad(Dims D, const uint16_t* __re
             for (int nb = 0; nb < NB; nb++)
 #pragma unroll
                 for (int kb = 0; kb < KB; kb++) {
-                    const s4 bq = {b[kb][q], b[kb][q + 1], b[kb][q + 2], b[kb][q + 3]};
+                    s4 bq = {b[kb][q], b[kb][q + 1], b[kb][q + 2], b[kb][q + 3]};
+                    if (TX > 1 && q == 0) {
+#pragma unroll
+                        for (int j = 0; j < 4; j++) bq[j] = xk + j < nx ? bq[j] : (short)0;
+                    }
                     acc[q][nb][kb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[nb], bq, acc[q][nb][kb], 0, 0, 0);
                 }
     }

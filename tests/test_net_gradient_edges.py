@@ -31,3 +31,34 @@ def test_gradients_at_the_splits():
                 e = np.linalg.norm(pg[name][k] - po[name][k]) / max(np.linalg.norm(po[name][k]), 1e-300)
                 assert e < 3e-2 or np.linalg.norm(po[name][k]) == 0 == np.linalg.norm(pg[name][k]), (shape, name, k, e)
     net.close()
+
+
+@pytest.mark.parametrize("nx", [17, 20, 31, 32])
+def test_infinity_in_a_rows_last_position(nx):
+    """An input of infinity at the end of a row, which the first layer's negative weights and its ReLU turn into 0:
+    the weight gradients of the taps that would pair it with a position past the row stay finite."""
+    from robtop_amd.learned import WarmStartNet
+    print(f"[learned] infinity at x = {nx - 1}", flush=True)
+    theta = on.random_params(21).astype(np.float32)
+    w = theta[:27 * 16 * 16].reshape(27, 16, 16)
+    w[:, :, 0] = -np.abs(w[:, :, 0]) - 0.01
+    net = WarmStartNet(0)
+    net.set_params(theta)
+    rng = np.random.default_rng(nx)
+    shape = (5, 6, nx)
+    x = rng.standard_normal(shape + (4,)).astype(np.float32)
+    x[2, 3, nx - 1, 0] = np.inf
+    t = rng.standard_normal(shape + (3,)).astype(np.float32)
+    loss, g = net.gradient(x, t)
+    with np.errstate(invalid="ignore"):
+        lo, go = on.loss_and_grad(theta.astype(np.float64), x.astype(np.float64), t.astype(np.float64), emulate=True)
+    assert np.isfinite(lo) and abs(loss - lo) / lo < 1e-3, (loss, lo)
+    pg, po = on.unpack(g), on.unpack(go)
+    for name in on.LAYERS:
+        wg, wo = pg[name][0], po[name][0]
+        if name == "E0A":
+            assert np.isfinite(wo[0::3]).all() and np.isnan(wo[1::3, :, 0]).any()
+            wg, wo = wg[0::3], wo[0::3]     # the taps at dx = -1
+        assert np.isfinite(wg).all(), name
+        assert np.linalg.norm(wg - wo) < 3e-2 * np.linalg.norm(wo), name
+    net.close()
