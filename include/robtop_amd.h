@@ -427,10 +427,10 @@ int rt_voxelize_mesh_noalloc(const float* d_coords, int nverts, const int* d_fac
 
 /* Autotuner (no counterpart in the reference): on this hierarchy's own sizes,
  * times each launch-shape alternative `reps` times with HIP events and keeps
- * the fastest: z planes per workgroup of the finest residual / apply (8 .. 48),
- * the finest smoother implementation (rt_set_fine_smoother), and per coarse
- * level the sliced (nine waves per 64 nodes) or thread-per-node smoother and
- * residual kernels. The operator is the same; only the summation order of a
+ * the fastest: z planes per workgroup of the finest residual / apply (1 .. 48; the
+ * value in use stays unless another is faster), the finest smoother implementation
+ * (rt_set_fine_smoother), and per coarse level the sliced (nine waves per 64 nodes)
+ * or thread-per-node smoother and residual kernels. The operator is the same; only the summation order of a
  * coarse node's 27 neighbour blocks differs between the two coarse kernel
  * forms (the finest-level choices are bit-identical). Needs rt_update_stencil first; uses the current force and
  * displacement as data. info[6] = {z planes, ms of residual + apply, smoother
