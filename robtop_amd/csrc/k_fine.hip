@@ -881,26 +881,36 @@ template void launch_fine_gs_sweep2<float>(const Geom&, Vec3<const float>, Vec3<
 template void launch_fine_gs_sweep2<double>(const Geom&, Vec3<const double>, Vec3<double>, Vec3<const double>,
                                             const float*, const uint8_t*, bool, bool, hipStream_t);
 
-// the row kernel's workgroup for a launch of `rows` rows (of all its vectors): rpw whole rows (0: too
-// long for it) of npr pairs in nt threads. Boxes are a multiple of the coarsest
-// spacing plus one node long, so a row's pairs often pass a multiple of 64 by
-// one. Where a launch fills the chip, the last pair's thread then takes the
-// even node left over as well (a wave of one lane would hold a fifth to a half
-// of the wave slots); where it does not, that would only lengthen the chain
-// (128 x 64 x 64 elements: 42.7 against 36.5 us a sweep). Other lengths put
-// several rows into a workgroup if that fills its lanes better and enough
-// workgroups remain.
+// the row kernel's workgroup for a launch of `rows` rows (of all its vectors): rpw
+// whole rows of npr pairs in nt threads, or rpw = 0 where the pair kernel takes the
+// launch: rows too long for a workgroup, and FP64 rows of five waves, which leave
+// three of a CU's eight wave slots empty (520 x 72 x 72 elements: 228 us a sweep, 192
+// by the pair kernel, 544 x 80 x 80 242 and 212; with nearly full lanes the two are
+// close: 600 x 64 x 64 141 and 142, 600 x 128 x 128 525 and 551).
+// Boxes are a multiple of the coarsest spacing plus one node long, so a row's pairs
+// often pass a multiple of 64 by one. The last pair's thread then takes the even
+// node left over as well where that puts more workgroups on a CU (row_fit): after
+// two, four or eight whole waves, and one or (FP32) three (512 x 96 x 96 elements:
+// 125 us a sweep, 164 with a wave of one lane; FP64 195 and 272). Where it does not,
+// it only lengthens the chain: 640 x 96 x 96 219 against 182 us, FP64 393 and 301, and
+// FP64 at 384 x 128 x 128 315 and 285; the same in launches that do not fill the
+// chip (128 x 64 x 64: 42.7 against 36.5 us). Other lengths put several rows into a
+// workgroup if that fills its lanes better and enough workgroups remain.
 struct RowShape { int rpw, nt, npr; };
+// workgroups of w waves that a CU holds: up to four waves of one share the wave
+// slots freely, more are placed evenly over the four SIMDs
+template <typename T> static int row_fit(int w) { return 4 * kRowWaves<T> / (w <= 4 ? w : (w + 3) / 4 * 4); }
 template <typename T>
 static RowShape row_shape(const Geom& g, long long rows) {
-    const int nxe = (g.n[0] + 1) / 2;
-    if (nxe > 1 && nxe % 64 == 1 && nxe - 1 <= kRowThreads && rows * (nxe / 64 + 1) > 4096)
+    const int nxe = (g.n[0] + 1) / 2, w = nxe / 64;
+    if (w > 0 && nxe % 64 == 1 && nxe - 1 <= kRowThreads && row_fit<T>(w) > row_fit<T>(w + 1) && rows * (w + 1) > 4096)
         return RowShape{1, nxe - 1, nxe - 1};
     RowShape best{0, 0, nxe};
     double eff = 0;
     for (int rpw = 1; rpw <= 8 && rpw * nxe <= kRowThreads; rpw++) {
         if (rpw > 1 && rows / rpw < 1024) break;
         const int nt = (rpw * nxe + 63) / 64 * 64;
+        if (sizeof(T) == 8 && nt == 5 * 64) continue;
         const double e = (double)(rpw * nxe) / nt;
         if (e > eff * 1.05) {
             eff = e;

@@ -82,3 +82,32 @@ def test_preconditioner_sweeps_equal_the_tiled_smoother(shape):
         out.append(hg.get_displacement())
     assert np.array_equal(out[0], out[1])
     hg.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shorter,longer,sizes", [((384, 64, 64), (448, 64, 64), (64,)),
+                                                  ((640, 64, 64), (700, 64, 64), (32, 64))])
+def test_a_shorter_row_takes_no_longer(shorter, longer, sizes):
+    """Rows of one pair more than three or five whole waves: the workgroup shape must not cost more than rows that are
+    longer still (a tenth for the timings' spread)."""
+    import robtop_amd as rt
+    from robtop_amd.workloads import box_bits
+    print(f"[rows] sweep times {shorter} {longer}", flush=True)
+    t = {}
+    for s in (shorter, longer):
+        R = cube_side(*s)
+        hg = rt.HierarchyGrid.genFromMesh(box_bits(R, *s), R)
+        hg.set_material(1e6, 0.4, 3.0)
+        hg.init_rho(0.4)
+        nx, ny, nz = hg[0].nodes
+        fixed = np.zeros((nz, ny, nx), bool)
+        fixed[:, :, 0] = True
+        hg.set_support(fixed.reshape(-1) & hg[0].masks()[1])
+        hg.update_stencil()
+        for bits in sizes:
+            hg.time_fine_sweep(bits, 20)
+            t[s, bits] = min(hg.time_fine_sweep(bits, 20) for _ in range(5))
+        hg.close()
+    print({k: round(1e3 * v, 1) for k, v in t.items()}, flush=True)
+    for bits in sizes:
+        assert t[shorter, bits] <= 1.1 * t[longer, bits], bits
