@@ -24,6 +24,8 @@
 // Measured: 4,131 unknowns (17 x 9 x 9 nodes: 26 launches for 65 blocks) 1.33
 // ms, 675 unknowns 0.32 ms; rocSOLVER's dpotrf and dpotri took 18 ms for the
 // two together, as much as the rest of a SIMP step at 64 x 32 x 32 elements.
+// Larger ones, where rt_set_coarse_direct_dofs admits them: 10,125 unknowns (112^3
+// elements) 9 ms against 83, 22,356 (36 rods) 64 ms against 481.
 // A workgroup owns one tile row I and up to kGjCols tiles of it: W_I is formed
 // once (as much work as one tile), each wave 16 rows of it, and goes to MFMA
 // operand order through LDS.

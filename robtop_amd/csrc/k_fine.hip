@@ -362,10 +362,10 @@ __global__ void __launch_bounds__(256) RT_GS_ATTR k_fine_gs_pair(Geom g, Vec3<T>
 // neighbour rows from the caches once instead of twice, and waits for memory
 // once. Same arithmetic per node and the same order, so the same bits.
 //
-// Bound: FP32 FMA issue (0.55 ms of a sweep at 511 x 256 x 256 elements) with
-// the latency of the row loads, which 4 waves per SIMD hide in part; the pass
-// per parity was bound by its reads from beyond L2, 1.48 GB a launch against
-// 0.89 now. Measured, ms per FP32 sweep: 511 x 256 x 256 1.03 -> 0.79, 256 x
+// Bound: VALU issue (at 511 x 256 x 256 elements 0.60 of a sweep's 0.79 ms, 0.48 of
+// it the 555 FMA a node) with the latency of the row loads, which 4 waves per SIMD
+// hide in part; the pass per parity was bound by its traffic beyond L2, 1.59 GB a
+// launch against 0.82 now. Measured, ms per FP32 sweep: 511 x 256 x 256 1.03 -> 0.79, 256 x
 // 128 x 128 0.156 -> 0.130, 128 x 64 x 64 0.041 -> 0.037; FP64 1.66 -> 1.20,
 // 0.195 -> 0.178, 0.049 -> 0.045. A spilled register or a fifth wave of one
 // lane (see row_shape) costs all of that: 5 waves per SIMD with 7 spilled

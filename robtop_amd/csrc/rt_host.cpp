@@ -485,7 +485,10 @@ static void build_tile_mask(Level& L) {
 // residual, us) at zc = 24 and at the zc this picks: 48 x 24 x 24 elements 42.6
 // and 6.3 (1), 64 x 32 x 32 65.9 and 7.1 (1), 128 x 64 x 64 44.9 and 19.2 (4),
 // 256 x 128 x 128 106.7 and 85.4 (12), 384 x 192 x 192 291 and 274 (8); 160^3
-// and 511 x 256 x 256 stay at 24.
+// and 511 x 256 x 256 stay at 24. Batched launches run the same planes, though
+// several vectors fill the chip with longer columns: a cycle of eight takes 0.20,
+// 0.28 and 1.16 ms at the three smallest sizes (1.35, 1.63 and 2.46 ms with 24
+// planes and a launch a vector).
 static int pick_zc(const Level& L) {
     int best = 24;
     long long least = -1;
@@ -977,7 +980,7 @@ static void factor_level(Hier& H, int li, DirectPlan& P, DBuf& Ainv, DBuf& rowsl
     RT_HIP(hipMemcpyAsync(&info, H.dinfo.p, sizeof(int), hipMemcpyDeviceToHost, H.s));
     RT_HIP(hipStreamSynchronize(H.s));
     if (info != 0)
-        throw std::domain_error("coarsest system: Cholesky factorisation failed (not positive definite; no supports?)");
+        throw std::domain_error("coarsest system: not positive definite (no supports?)");
     if (singular) {
         // M <- P M P = M - G R^T - R G^T + R (R^T G) R^T, G = M R
         const double* R = Rd_.as<double>();
@@ -2722,11 +2725,13 @@ static void worst_apply(Hier& H, const double* q, double* y, double solve_tol, i
 
 // ---------------------------------------------------------------------------
 // Batched solves for the worst-case search: nb <= kBatchMax right-hand sides
-// through one preconditioner cycle. Every kernel of the cycle and of the CG
-// takes all vectors in one launch: a vector of a small or middling grid does not
-// fill the chip by itself, and the launches of eight cost eight times their
-// latency (block Lanczos on a 128^3 torus: 155 ms with the finest level's and the
-// CG's kernels launched per vector, 99 ms so). The coarser levels read each
+// through one preconditioner cycle. The kernels of the cycle and of the CG take
+// all vectors in one launch: a vector of a small or middling grid does not fill
+// the chip by itself, and the launches of eight cost eight times their latency
+// (block Lanczos on a 128^3 torus: 155 ms with the finest level's and the CG's
+// kernels launched per vector, 99 ms so). Once per vector run the correction of
+// floating clusters, the tiled smoother where that is chosen, and at residual
+// replacements the subtraction and the flush of the solution increment. The coarser levels read each
 // stencil coefficient once for all nb vectors, and the coarsest applies its
 // inverse to all nb at once. The whole batched cycle is captured into one HIP
 // graph. No counterpart in the reference, which solves one load at a time
