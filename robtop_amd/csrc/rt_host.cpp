@@ -1430,8 +1430,8 @@ static void pcg_reliable(Hier& H, double tol, int maxit, int pre, int post, rt_s
             launch_sum_partials(H.partials.as<double>(), ns, H.cg(kCgRr), H.s);
             CgValues v;
             cg_read(H, v);
-            if (!(v[kCgPq][0] > 0)) throw std::domain_error("PCG breakdown: p.Ap <= 0");
             if (it > 1) H.cg_beta.push_back(v[kCgBeta][0]);
+            if (!(v[kCgPq][0] > 0)) throw std::domain_error("PCG breakdown: p.Ap <= 0");
             apend = v[kCgAlpha][0];
             H.cg_alpha.push_back(apend);
             flushed = false;

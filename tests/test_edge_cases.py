@@ -86,3 +86,23 @@ def test_solver_state_errors():
     assert L.rt_net_train(net.handle, 1, 1, ctypes.c_float(1e-3), ctypes.c_uint64(0), None) == _lib.RT_ESTATE
     net.close()
     hg.close()
+
+
+@pytest.mark.gpu
+def test_coefficients_after_a_breakdown():
+    """One element of negative stiffness: the solve ends where p.Ap is not positive, with the direction's coefficient of
+    every completed iteration on record (the last one led to the direction that broke down)."""
+    import robtop_amd as rt
+    from bench import build_problem
+    print("[edge] breakdown", flush=True)
+    hg, bits, R, fixed, f, rho = build_problem(64, 32, 32, 3)
+    r = rho.copy()
+    r[len(r) // 2 + 1000] = -0.5
+    hg.set_density(r)
+    hg.update_stencil()
+    hg.set_displacement(np.zeros_like(f))
+    with pytest.raises(rt.RobtopError, match="breakdown"):
+        hg.solve(tol=1e-6, maxit=50, mode=rt.RT_SOLVE_RELIABLE)
+    a, b = hg.cg_coefficients()
+    assert len(a) > 0 and (a > 0).all() and (b != 0).all()
+    hg.close()
