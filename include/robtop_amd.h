@@ -428,7 +428,7 @@ int rt_voxelize_mesh_noalloc(const float* d_coords, int nverts, const int* d_fac
 /* Autotuner (no counterpart in the reference): on this hierarchy's own sizes,
  * times each launch-shape alternative `reps` times with HIP events and keeps
  * the fastest: z planes per workgroup of the finest residual / apply (1 .. 48; the
- * value in use stays unless another is faster), the finest smoother implementation
+ * value in use stays unless another is 5 % faster), the finest smoother implementation
  * (rt_set_fine_smoother), and per coarse level the sliced (nine waves per 64 nodes)
  * or thread-per-node smoother and residual kernels. The operator is the same; only the summation order of a
  * coarse node's 27 neighbour blocks differs between the two coarse kernel
