@@ -65,8 +65,9 @@ __device__ __forceinline__ double gj_rcp(double x) {
 // pivot columns, which their 16 threads put into LDS. 4 x 4 blocks, since the
 // LDS reads of the pivot columns are what a step takes: 8 values a thread and
 // column against 17 with a thread per row.
-// The pivot block is scaled by a power of two (exact) so that its determinant is
-// in range for every stiffness whose inverse is.
+// A pivot block's determinant is formed times a power of two (exact; lane l of a
+// wave keeps that of pivots 2 l, 2 l + 1, from the tile's diagonal before the
+// sweeps), so that it is in range for every stiffness whose inverse is.
 __device__ __forceinline__ void gj_invert(const double (*S)[GB + 1], double (*col)[2][GB], double* __restrict__ D,
                                           int* __restrict__ info) {
     const int ti = threadIdx.x >> 4, tj = threadIdx.x & 15;
@@ -75,6 +76,8 @@ __device__ __forceinline__ void gj_invert(const double (*S)[GB + 1], double (*co
     for (int i = 0; i < 4; i++)
 #pragma unroll
         for (int j = 0; j < 4; j++) a[i][j] = S[4 * ti + i][4 * tj + j];
+    const int dg = 2 * (threadIdx.x & 31);
+    const int sc_hi = (1023 - min(max(__builtin_amdgcn_frexp_exp(S[dg][dg]), -1000), 1000)) << 20;
     bool bad = false;
     for (int tp = 0; tp < 16; tp++) {
 #pragma unroll
@@ -86,19 +89,18 @@ __device__ __forceinline__ void gj_invert(const double (*S)[GB + 1], double (*co
                 for (int i = 0; i < 4; i++) { c[0][4 * ti + i] = a[i][2 * h]; c[1][4 * ti + i] = a[i][2 * h + 1]; }
             }
             __syncthreads();
-            const double t00 = c[0][p];
-            const int sx = -__builtin_amdgcn_frexp_exp(t00);
-            const double d00 = __builtin_ldexp(t00, sx), d01 = __builtin_ldexp(c[1][p], sx),
-                         d11 = __builtin_ldexp(c[1][p + 1], sx);
+            const double d00 = c[0][p], d01 = c[1][p], d11 = c[1][p + 1];
+            const double sc = __hiloint2double(__builtin_amdgcn_readlane(sc_hi, 2 * tp + h), 0);
+            const double s00 = d00 * sc, s01 = d01 * sc, s11 = d11 * sc;
             double r0[4], r1[4], k0[4], k1[4];
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 r0[i] = c[0][4 * ti + i]; r1[i] = c[1][4 * ti + i];
                 k0[i] = c[0][4 * tj + i]; k1[i] = c[1][4 * tj + i];
             }
-            const double det = d00 * d11 - d01 * d01;
+            const double det = s00 * d11 - s01 * d01;                    // times sc, as the others
             bad = bad || !(d00 > 0) || !(det > 0);
-            const double rd = __builtin_ldexp(gj_rcp(det), sx), e00 = d11 * rd, e01 = -d01 * rd, e11 = d00 * rd;
+            const double rd = gj_rcp(det), e00 = s11 * rd, e01 = -s01 * rd, e11 = s00 * rd;
             double x0[4], x1[4];
 #pragma unroll
             for (int i = 0; i < 4; i++) {                                // W
